@@ -86,18 +86,33 @@ __device__ __forceinline__ float psum(const float (&a)[N]) {
   return psum_tree(r);
 }
 
-// The same sum over G lanes (one value per lane, G = 8 or 16) as an xor
-// butterfly: xor 8 forms r[j] = a[j] + a[j+8], then xor 1, 2, 4 build the tree.
-// IEEE addition is commutative, so every lane of the group ends with the
-// identical, numpy-ordered result.
+// v of another lane of the same 16-lane row, by a DPP move: ror 8 (the lane whose index
+// differs in bit 3), quad permutations (bit 0, bit 1) and the half-row mirror (lane 7 - i of
+// each 8). Cross-lane steps on the VALU: no LDS round trip, as __shfl_xor (ds_bpermute) takes.
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor8 = 0x128;
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  const int i = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, i, CTRL, 0xF, 0xF, true));
+}
+
+// v over the 8 lanes of an aligned lane octet, as the tree ((v0+v1)+(v2+v3))+((v4+v5)+(v6+v7)),
+// in every lane. After the first two steps the four lanes of a quad hold one value, so the
+// half-row mirror reads the other quad's, as an xor by 4 would.
+__device__ __forceinline__ float tree8(float v) {
+  v = v + dpp<kDppXor1>(v);
+  v = v + dpp<kDppXor2>(v);
+  return v + dpp<kDppHalfMirror>(v);
+}
+
+// psum over G lanes (one value per lane, G = 8 or 16): lanes j and j + 8 form r[j] = a[j] +
+// a[j+8], then tree8. IEEE addition is commutative, so every lane of the group ends with the
+// identical, numpy-ordered result. All 64 lanes must be active.
 template <int G>
 __device__ __forceinline__ float gsum(float v) {
   static_assert(G == 8 || G == 16, "group width");
-  if (G == 16) v = v + __shfl_xor(v, 8);
-  v = v + __shfl_xor(v, 1);
-  v = v + __shfl_xor(v, 2);
-  v = v + __shfl_xor(v, 4);
-  return 0.0f + v;
+  if (G == 16) v = v + dpp<kDppRor8>(v);
+  return 0.0f + tree8(v);
 }
 
 template <int G>

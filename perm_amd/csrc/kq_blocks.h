@@ -7,8 +7,9 @@
 // ones of Q4_K and Q5_K). Sub-block fits run in-lane on registers; superblock-level
 // steps (maxima, super-scale fits, the 256-wide sum of squares) run across the
 // G lanes of the superblock with xor-butterfly reductions that reproduce
-// numpy's pairwise order. Codes and per-superblock fields are staged in LDS
-// and the wave's contiguous output bytes leave as coalesced dword stores.
+// numpy's pairwise order. What leaves (KqOut) is the container bytes, the scale fields
+// alone (the EF commits, whose code bytes the repack writes), or the decoded weights
+// (the PERM objective, which needs no bytes).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -48,10 +49,13 @@ struct Kq<CP_Q6_K> {
 //  Q3_K: a[k] = 6-bit scale 0..63
 //  Q4_K, Q5_K: a[0..7] = 6-bit scales, a[8..15] = 6-bit mins
 //  Q6_K: a[k] = int8 scale
-struct SbFields {
+struct alignas(4) SbFields {
   uint8_t a[16];
   uint16_t d, dmin;
 };
+
+// What an encode leaves in memory.
+enum class KqOut { kBytes, kFields, kRecon };
 
 // numpy's pairwise sum of a superblock's 256 values staged in LDS, computed by
 // the G lanes of the superblock: split 128 + 128, each half with 8 sequential
@@ -63,11 +67,8 @@ __device__ __forceinline__ float sum256_lds(const float* a, int g) {
     float r = p[0];
 #pragma unroll
     for (int m = 1; m < 16; ++m) r = r + p[8 * m];
-    r = r + __shfl_xor(r, 1);
-    r = r + __shfl_xor(r, 2);
-    r = r + __shfl_xor(r, 4);
-    float tot = r + __shfl_xor(r, 8);
-    return 0.0f + tot;
+    r = tree8(r);
+    return 0.0f + (r + dpp<kDppRor8>(r));
   } else {
     float r0 = a[g], r1 = a[128 + g];
 #pragma unroll
@@ -75,96 +76,144 @@ __device__ __forceinline__ float sum256_lds(const float* a, int g) {
       r0 = r0 + a[g + 8 * m];
       r1 = r1 + a[128 + g + 8 * m];
     }
-    r0 = r0 + __shfl_xor(r0, 1);
-    r1 = r1 + __shfl_xor(r1, 1);
-    r0 = r0 + __shfl_xor(r0, 2);
-    r1 = r1 + __shfl_xor(r1, 2);
-    r0 = r0 + __shfl_xor(r0, 4);
-    r1 = r1 + __shfl_xor(r1, 4);
-    return 0.0f + (r0 + r1);
+    return 0.0f + (tree8(r0) + tree8(r1));
   }
 }
 
-// One output byte of a packed superblock from its staged codes and fields
-// (ggml block layouts; kquant.py:407-413, :474-485, :565-571, :664-677).
-template <int TT>
-__device__ __forceinline__ uint32_t pack_byte(const uint8_t* c, const SbFields& f, int b) {
-  if constexpr (TT == CP_Q2_K) {
-    if (b < 16) return f.a[b];
-    if (b < 80) {
-      int k = b - 16, base = (k >> 5) * 128 + (k & 31);
-      return c[base] | c[base + 32] << 2 | c[base + 64] << 4 | c[base + 96] << 6;
-    }
-    if (b < 82) return (f.d >> (8 * (b - 80))) & 0xFF;
-    return (f.dmin >> (8 * (b - 82))) & 0xFF;
-  } else if constexpr (TT == CP_Q3_K) {
-    if (b < 32) {
-      uint32_t m = 0;
+// Items 0 .. C - 1 of each of a wave's S superblocks, handed to its lanes: f(superblock, item).
+template <int S, int C, class F>
+__device__ __forceinline__ void wave_items(int lane, const F& f) {
+  static_assert((C & (C - 1)) == 0, "power of two per superblock");
 #pragma unroll
-      for (int j = 0; j < 8; ++j) m |= ((c[32 * j + b] >> 2) & 1u) << j;
-      return m;
-    }
-    if (b < 96) {
-      int k = b - 32, base = (k >> 5) * 128 + (k & 31);
-      return (c[base] & 3) | (c[base + 32] & 3) << 2 | (c[base + 64] & 3) << 4 |
-             (c[base + 96] & 3) << 6;
-    }
-    if (b < 108) {
-      int m = b - 96;
-      if (m < 8) return (f.a[m] & 0xF) | (f.a[m + 8] & 0xF) << 4;
-      m -= 8;
-      uint32_t v = 0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v |= ((uint32_t)(f.a[m + 4 * q] >> 4) & 3u) << (2 * q);
-      return v;
-    }
-    return (f.d >> (8 * (b - 108))) & 0xFF;
-  } else if constexpr (TT == CP_Q4_K || TT == CP_Q5_K) {
-    if (b < 2) return (f.d >> (8 * b)) & 0xFF;
-    if (b < 4) return (f.dmin >> (8 * (b - 2))) & 0xFF;
-    if (b < 16) {
-      int m = b - 4;
-      if (m < 4) return (f.a[m] | (f.a[m + 4] >> 4) << 6) & 0xFF;
-      if (m < 8) return (f.a[8 + m - 4] | (f.a[8 + m] >> 4) << 6) & 0xFF;
-      return (f.a[m - 4] & 0xF) | (f.a[8 + m - 4] & 0xF) << 4;
-    }
-    constexpr int body = TT == CP_Q5_K ? 48 : 16;
-    if (TT == CP_Q5_K && b < body) {
-      // qh: bit 2c of byte j is code (64c + j) >= 16, bit 2c+1 is code (64c + 32 + j) >= 16
-      int j = b - 16;
-      uint32_t v = 0;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) v |= (uint32_t)(c[32 * q + j] >> 4) << q;
-      return v;
-    }
-    int k = b - body, base = (k >> 5) * 64 + (k & 31);
-    return (c[base] & 0xF) | (c[base + 32] & 0xF) << 4;
-  } else {  // Q6_K
-    if (b < 128) {
-      int h = b >> 6, k = b & 63;
-      int base = h * 128 + (k & 31) + (k >= 32 ? 32 : 0);
-      return (c[base] & 0xF) | (c[base + 64] & 0xF) << 4;
-    }
-    if (b < 192) {
-      int k = b - 128, base = (k >> 5) * 128 + (k & 31);
-      return (c[base] >> 4) | (c[base + 32] >> 4) << 2 | (c[base + 64] >> 4) << 4 |
-             (c[base + 96] >> 4) << 6;
-    }
-    if (b < 208) return f.a[b - 192];
-    return (f.d >> (8 * (b - 208))) & 0xFF;
+  for (int i0 = 0; i0 < S * C; i0 += 64) {
+    const int i = i0 + lane;
+    if (S * C - i0 >= 64 || i < S * C) f(i / C, i % C);
   }
+}
+
+// The packed superblocks of a wave (ggml block layouts; kquant.py:407-413, :474-485,
+// :565-571, :664-677): its S superblocks of BP bytes at dst, four bytes per item from four
+// codes at a time (the codes of a superblock are consecutive LDS bytes, so one LDS word holds
+// the codes of four output bytes). Packed byte by byte, each byte chosen among the fields by
+// its offset, this was a fifth of the Q6_K encode's instructions (divergent branches and one
+// LDS byte read per code). Superblocks from nvalid on are left out. CODES false: the scale
+// fields alone.
+template <int TT, bool CODES>
+__device__ __forceinline__ void pack_wave(const uint8_t* codes, const SbFields* f, int lane,
+                                          int nvalid, uint8_t* dst) {
+  constexpr int S = 64 / Kq<TT>::G, BP = Kq<TT>::BP;
+  constexpr uint32_t M1 = 0x01010101u, M3 = 0x03030303u, MF = 0x0F0F0F0Fu;
+  const auto c = [&](int s, int k) { return *reinterpret_cast<const uint32_t*>(codes + s * 256 + k); };
+  const auto a = [&](int s, int w) { return *reinterpret_cast<const uint32_t*>(f[s].a + 4 * w); };
+  const auto put = [&](int s, int off, uint32_t v) {  // four bytes at a 2- or 4-byte boundary
+    if (s >= nvalid) return;
+    uint8_t* p = dst + s * BP + off;
+    if constexpr (BP % 4 == 0) {
+      *reinterpret_cast<uint32_t*>(p) = v;
+    } else {
+      reinterpret_cast<uint16_t*>(p)[0] = (uint16_t)v;
+      reinterpret_cast<uint16_t*>(p)[1] = (uint16_t)(v >> 16);
+    }
+  };
+  const auto put_d = [&](int off) {  // the lone fp16 d of the types without mins
+    if (lane < S && lane < nvalid) *reinterpret_cast<uint16_t*>(dst + lane * BP + off) = f[lane].d;
+  };
+  if constexpr (TT == CP_Q2_K) {
+    if constexpr (CODES)
+      wave_items<S, 16>(lane, [&](int s, int j) {
+        const int k = (j >> 3) * 128 + 4 * (j & 7);
+        put(s, 16 + 4 * j, c(s, k) | c(s, k + 32) << 2 | c(s, k + 64) << 4 | c(s, k + 96) << 6);
+      });
+    wave_items<S, 4>(lane, [&](int s, int j) { put(s, 4 * j, a(s, j)); });
+    wave_items<S, 1>(lane, [&](int s, int) { put(s, 80, (uint32_t)f[s].d | (uint32_t)f[s].dmin << 16); });
+  } else if constexpr (TT == CP_Q3_K) {
+    if constexpr (CODES) {
+      wave_items<S, 8>(lane, [&](int s, int j) {
+        uint32_t v = 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v |= ((c(s, 32 * q + 4 * j) >> 2) & M1) << q;
+        put(s, 4 * j, v);
+      });
+      wave_items<S, 16>(lane, [&](int s, int j) {
+        const int k = (j >> 3) * 128 + 4 * (j & 7);
+        put(s, 32 + 4 * j, (c(s, k) & M3) | (c(s, k + 32) & M3) << 2 | (c(s, k + 64) & M3) << 4 |
+                               (c(s, k + 96) & M3) << 6);
+      });
+    }
+    wave_items<S, 4>(lane, [&](int s, int j) {
+      const uint32_t w0 = a(s, 0), w1 = a(s, 1), w2 = a(s, 2), w3 = a(s, 3);
+      if (j == 0) put(s, 96, (w0 & MF) | (w2 & MF) << 4);
+      if (j == 1) put(s, 100, (w1 & MF) | (w3 & MF) << 4);
+      if (j == 2)
+        put(s, 104, ((w0 >> 4) & M3) | ((w1 >> 4) & M3) << 2 | ((w2 >> 4) & M3) << 4 | ((w3 >> 4) & M3) << 6);
+    });
+    put_d(108);
+  } else if constexpr (TT == CP_Q4_K || TT == CP_Q5_K) {
+    constexpr int body = TT == CP_Q5_K ? 48 : 16;
+    if constexpr (CODES) {
+      if constexpr (TT == CP_Q5_K)  // qh: bit q of byte j is code (32q + j) >= 16
+        wave_items<S, 8>(lane, [&](int s, int j) {
+          uint32_t v = 0;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v |= ((c(s, 32 * q + 4 * j) >> 4) & M1) << q;
+          put(s, 16 + 4 * j, v);
+        });
+      wave_items<S, 32>(lane, [&](int s, int j) {
+        const int k = (j >> 3) * 64 + 4 * (j & 7);
+        put(s, body + 4 * j, (c(s, k) & MF) | (c(s, k + 32) & MF) << 4);
+      });
+    }
+    wave_items<S, 4>(lane, [&](int s, int j) {
+      const uint32_t s0 = a(s, 0), s1 = a(s, 1), m0 = a(s, 2), m1 = a(s, 3);
+      put(s, 4 * j, j == 0   ? (uint32_t)f[s].d | (uint32_t)f[s].dmin << 16
+                    : j == 1 ? s0 | ((s1 >> 4) & M3) << 6
+                    : j == 2 ? m0 | ((m1 >> 4) & M3) << 6
+                             : (s1 & MF) | (m1 & MF) << 4);
+    });
+  } else {  // Q6_K
+    if constexpr (CODES) {
+      wave_items<S, 32>(lane, [&](int s, int j) {
+        const int k = (j >> 4) * 128 + 4 * (j & 15);
+        put(s, 4 * j, (c(s, k) & MF) | (c(s, k + 64) & MF) << 4);
+      });
+      wave_items<S, 16>(lane, [&](int s, int j) {
+        const int k = (j >> 3) * 128 + 4 * (j & 7);
+        put(s, 128 + 4 * j, ((c(s, k) >> 4) & M3) | ((c(s, k + 32) >> 4) & M3) << 2 |
+                                ((c(s, k + 64) >> 4) & M3) << 4 | ((c(s, k + 96) >> 4) & M3) << 6);
+      });
+    }
+    wave_items<S, 4>(lane, [&](int s, int j) { put(s, 192 + 4 * j, a(s, j)); });
+    put_d(208);
+  }
+}
+
+// LDS writes of this wave's lanes before its later LDS reads (the LDS serves one wave's
+// accesses in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Encode the superblocks of block ``blk`` (kWavesPerBlock waves of S
 // superblocks each) of one [NB superblocks] tensor; nsb superblocks per row.
-template <int TT, bool IMAT>
+// OUT: kBytes and kFields write container bytes to ``out``; kRecon writes the decoded
+// float32 weights to ``recon`` and no bytes.
+template <int TT, bool IMAT, KqOut OUT = KqOut::kBytes>
 __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
                                                 const float* __restrict__ qw, int64_t NB,
                                                 int64_t nsb, uint8_t* __restrict__ out,
-                                                int64_t blk) {
+                                                int64_t blk, float* __restrict__ recon = nullptr) {
   constexpr int G = Kq<TT>::G, SUBW = Kq<TT>::SUBW, BP = Kq<TT>::BP, S = 64 / G;
-  __shared__ float s_sq[IMAT ? kWavesPerBlock : 1][IMAT ? S * 256 : 1];
-  __shared__ uint8_t s_codes[kWavesPerBlock][S * 256];
+  // one buffer per wave: the squares of the weighted path, then the packed bytes or the
+  // decoded weights on their way out
+  constexpr bool kSquares = IMAT && TT != CP_Q6_K;
+  constexpr int kOutBytes = OUT == KqOut::kBytes ? (S * BP + 15) / 16 * 16
+                            : OUT == KqOut::kRecon ? S * 256 * 4 : 16;
+  constexpr int kBufBytes = kSquares && S * 256 * 4 > kOutBytes ? S * 256 * 4 : kOutBytes;
+  __shared__ __align__(16) uint8_t s_buf[kWavesPerBlock][kBufBytes];
+  __shared__ __align__(16) uint8_t s_codes[OUT == KqOut::kBytes ? kWavesPerBlock : 1]
+                                          [OUT == KqOut::kBytes ? S * 256 : 16];
   __shared__ SbFields s_f[kWavesPerBlock][S];
   // the make_qp_quants problems of the weighted affine types: two per superblock
   constexpr bool kQp = IMAT && (TT == CP_Q2_K || TT == CP_Q4_K || TT == CP_Q5_K);
@@ -192,8 +241,8 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
 
   // importance weights qw * sqrt(k*sum(x^2)/256 + x^2)  (kquant.py:380-383, :453-455, :537-539)
   float wt[SUBW];
-  if constexpr (IMAT && TT != CP_Q6_K) {
-    float* sq = &s_sq[wv][sl * 256];
+  if constexpr (kSquares) {
+    float* sq = reinterpret_cast<float*>(s_buf[wv]) + sl * 256;
 #pragma unroll
     for (int i = 0; i < SUBW; ++i) sq[g * SUBW + i] = xv[i] * xv[i];
     __syncthreads();
@@ -221,6 +270,7 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
   }
 
   int L[SUBW];
+  float rdl = 0.0f, rml = 0.0f;  // the decoders' sub-block step and offset (kRecon)
   SbFields& F = s_f[wv][sl];
 
   if constexpr (TT == CP_Q2_K) {
@@ -248,11 +298,17 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
     }
     uint16_t d16 = half_bits(d), m16 = half_bits(dmin);
     float dl = half_value(d16) * (float)sc_i, ml = half_value(m16) * (float)mn_i;
-    if (dl != 0.0f) {
+    if constexpr (OUT != KqOut::kFields) {
+      if (dl != 0.0f) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) L[i] = clampi(rint_magic((xv[i] + ml) / dl), 0, 3);
-    } else {
-      affine_final_codes<16>(xv, fit, 3, L);  // the search's codes stay where dl == 0
+        for (int i = 0; i < 16; ++i) L[i] = clampi(rint_magic((xv[i] + ml) / dl), 0, 3);
+      } else {
+        affine_final_codes<16>(xv, fit, 3, L);  // the search's codes stay where dl == 0
+      }
+    }
+    if constexpr (OUT == KqOut::kRecon) {
+      rdl = half_value(d16) * (float)(sc_i & 0xF);
+      rml = half_value(m16) * (float)(mn_i & 0xF);
     }
     F.a[g] = (uint8_t)((sc_i & 0xF) | (mn_i & 0xF) << 4);
     if (g == 0) {
@@ -262,10 +318,11 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
   } else if constexpr (TT == CP_Q3_K) {
     int Ls;
     float d;
+    SignedFit fit;
     if constexpr (IMAT) {
-      float scale = fit_signed<16>(xv, wt, 4, L);
+      fit = fit_signed<16>(xv, wt, kQxQ3);
       float sw = psum<16>(wt);
-      d = gfit_signed<16>(scale, sw, 32, g, &Ls);
+      d = gfit_signed<16>(fit.scale, sw, 32, g, &Ls);
     } else {
       float scale = fit_signed_descent16(xv, 4, L);
       float amax;
@@ -278,10 +335,18 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
     }
     uint16_t d16 = half_bits(d);
     float dsub = half_value(d16) * (float)(Ls - 32);
-    if (dsub != 0.0f) {
+    if constexpr (OUT != KqOut::kFields) {
+      if constexpr (IMAT) {
+        if (dsub != 0.0f)
+          signed_requant<16>(xv, fit, dsub, 4, L);
+        else
+          signed_final_codes<16>(xv, fit, 4, L);  // the search's codes stay where dsub == 0
+      } else if (dsub != 0.0f) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) L[i] = clampi(rint_magic(xv[i] / dsub), -4, 3) + 4;
+        for (int i = 0; i < 16; ++i) L[i] = clampi(rint_magic(xv[i] / dsub), -4, 3) + 4;
+      }
     }
+    if constexpr (OUT == KqOut::kRecon) rdl = half_value(d16) * (float)((Ls & 63) - 32);
     F.a[g] = (uint8_t)Ls;
     if (g == 0) F.d = d16;
   } else if constexpr (TT == CP_Q4_K || TT == CP_Q5_K) {
@@ -327,11 +392,17 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
     }
     uint16_t d16 = half_bits(d), m16 = half_bits(dmin);
     float dl = half_value(d16) * (float)Ls, ml = half_value(m16) * (float)Lm;
-    if (dl != 0.0f) {
+    if constexpr (OUT != KqOut::kFields) {
+      if (dl != 0.0f) {
 #pragma unroll
-      for (int i = 0; i < 32; ++i) L[i] = clampi(rint_magic((xv[i] + ml) / dl), 0, TOP);
-    } else {
-      affine_final_codes<32>(xv, fit, TOP, L);  // the search's codes stay where dl == 0
+        for (int i = 0; i < 32; ++i) L[i] = clampi(rint_magic((xv[i] + ml) / dl), 0, TOP);
+      } else {
+        affine_final_codes<32>(xv, fit, TOP, L);  // the search's codes stay where dl == 0
+      }
+    }
+    if constexpr (OUT == KqOut::kRecon) {
+      rdl = half_value(d16) * (float)(Ls & 63);
+      rml = half_value(m16) * (float)(Lm & 63);
     }
     F.a[g] = (uint8_t)Ls;
     F.a[8 + g] = (uint8_t)Lm;
@@ -344,30 +415,59 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
 #pragma unroll
       for (int i = 0; i < 16; ++i) wt[i] = xv[i] * xv[i];
     }
-    float scale = fit_signed<16>(xv, wt, 32, L);
+    const SignedFit fit = fit_signed<16>(xv, wt, kQxQ6);
     float amax;
-    float smax = gfirst_absmax<16>(scale, g, &amax);
+    float smax = gfirst_absmax<16>(fit.scale, g, &amax);
     bool dead = amax < 1e-15f;
     float is = -128.0f / (dead ? 1.0f : smax);
     float d = 1.0f / is;
-    int q = rint_magic(is * scale);
+    int q = rint_magic(is * fit.scale);
     int8_t sc = (int8_t)(q < 127 ? q : 127);
     uint16_t d16 = half_bits(dead ? 0.0f : d);
     float dsub = half_value(d16) * (float)sc;
-    if (dsub != 0.0f && !dead) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) L[i] = clampi(rint_magic(xv[i] / dsub), -32, 31) + 32;
+    if constexpr (OUT != KqOut::kFields) {
+      if (dsub != 0.0f && !dead)
+        signed_requant<16>(xv, fit, dsub, 32, L);
+      else
+        signed_final_codes<16>(xv, fit, 32, L);  // the search's codes stay where dsub == 0
     }
     if (dead) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) L[i] = 0;
       sc = 0;
     }
+    if constexpr (OUT == KqOut::kRecon) rdl = half_value(d16) * (float)sc;
     F.a[g] = (uint8_t)sc;
     if (g == 0) F.d = d16;
   }
 
-  {
+  const int nvalid = sb0 >= NB ? 0 : (int)((NB - sb0) < S ? (NB - sb0) : S);
+  // what follows exchanges data between the lanes of one wave only
+  if constexpr (OUT == KqOut::kRecon) {
+    // y = (d*sc)*q - (dmin*m), the decoders' expression; each store writes 1 KB
+    constexpr int kOff = TT == CP_Q3_K ? 4 : TT == CP_Q6_K ? 32 : 0;
+    constexpr bool kMin = TT == CP_Q2_K || TT == CP_Q4_K || TT == CP_Q5_K;
+    float* o = reinterpret_cast<float*>(s_buf[wv]);
+    wave_lds_fence();
+#pragma unroll
+    for (int i = 0; i < SUBW; i += 4) {
+      float r[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float v = rdl * (float)(L[i + k] - kOff);
+        r[k] = kMin ? v - rml : v;
+      }
+      *reinterpret_cast<float4*>(o + lane * SUBW + i) = make_float4(r[0], r[1], r[2], r[3]);
+    }
+    wave_lds_fence();
+    float4* y = reinterpret_cast<float4*>(recon + sb0 * 256);
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+      if (i < nvalid) y[64 * i + lane] = reinterpret_cast<const float4*>(o)[64 * i + lane];
+  } else if constexpr (OUT == KqOut::kFields) {
+    wave_lds_fence();
+    pack_wave<TT, false>(nullptr, s_f[wv], lane, nvalid, out + sb0 * BP);
+  } else {
     uint8_t* c = &s_codes[wv][sl * 256 + g * SUBW];
 #pragma unroll
     for (int i = 0; i < SUBW; i += 4) {
@@ -375,27 +475,17 @@ __device__ __forceinline__ void kq_encode_block(const float* __restrict__ x,
                    (uint32_t)(L[i + 2] & 0xFF) << 16 | (uint32_t)(L[i + 3] & 0xFF) << 24;
       *reinterpret_cast<uint32_t*>(c + i) = v;
     }
-  }
-  __syncthreads();
-
-  if (sb0 >= NB) return;
-  const int nvalid = (int)((NB - sb0) < S ? (NB - sb0) : S);
-  const int bytes = nvalid * BP;
-  uint8_t* dst = out + sb0 * BP;
-  for (int dw = lane; dw < bytes / 4; dw += 64) {
-    uint32_t v = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      int bi = dw * 4 + k, s = bi / BP, b = bi - s * BP;
-      v |= pack_byte<TT>(&s_codes[wv][s * 256], s_f[wv][s], b) << (8 * k);
-    }
-    reinterpret_cast<uint32_t*>(dst)[dw] = v;
-  }
-  if ((bytes & 3) && lane == 0) {
-    int bi = bytes - 2, s = bi / BP, b = bi - s * BP;
-    uint32_t v = pack_byte<TT>(&s_codes[wv][s * 256], s_f[wv][s], b) |
-                 pack_byte<TT>(&s_codes[wv][s * 256], s_f[wv][s], b + 1) << 8;
-    *reinterpret_cast<uint16_t*>(dst + bi) = (uint16_t)v;
+    wave_lds_fence();
+    uint8_t* pk = s_buf[wv];
+    pack_wave<TT, true>(s_codes[wv], s_f[wv], lane, S, pk);
+    wave_lds_fence();
+    // the wave's contiguous bytes leave as coalesced dword stores
+    const int bytes = nvalid * BP;
+    uint8_t* dst = out + sb0 * BP;
+    for (int dw = lane; dw < bytes / 4; dw += 64)
+      reinterpret_cast<uint32_t*>(dst)[dw] = reinterpret_cast<const uint32_t*>(pk)[dw];
+    if ((bytes & 3) && lane == 0)
+      reinterpret_cast<uint16_t*>(dst)[bytes / 2 - 1] = reinterpret_cast<const uint16_t*>(pk)[bytes / 2 - 1];
   }
 }
 

@@ -2,7 +2,7 @@
 //
 // In-lane fits (one lane owns one sub-block of N values in registers):
 //   fit_affine<N, NUMS> make_qkx2 / make_qkx3 search      coldpress/kquant.py:42-94
-//   fit_signed<N>       make_qx_quants, rmse_type 1        coldpress/kquant.py:97-133
+//   fit_signed<N, NUMS> make_qx_quants, rmse_type 1        coldpress/kquant.py:97-133
 //   fit_signed_descent  make_q3_quants                     coldpress/kquant.py:136-179
 // Cross-lane fits (one lane owns one element of a G-wide vector of super-block
 // scales; G = 16 for Q2_K/Q3_K, 8 for Q4_K):
@@ -193,15 +193,72 @@ __device__ __forceinline__ AffineFit fit_affine(const float (&x)[N], const float
   return AffineFit{dead ? 0.0f : scale, -lo, best_inv, best_lo, dead};
 }
 
-// Symmetric signed fit x ~ scale * L, L in [-nmax, nmax-1]; weights w (pass
-// x*x for the unweighted path). L receives codes + nmax.
+// The candidate numerators -(nmax + 0.1 s), s = -9 .. 9 without 0, of make_qx_quants
+// (kquant.py:117-118), evaluated at compile time in float32 as the device would: the
+// product and the sum rounded once each, the negation exact.
+template <int NMAX>
+struct QxNums {
+  static constexpr int kNmax = NMAX, kSteps = 18;
+  float v[kSteps];
+  constexpr QxNums() : v() {
+    for (int k = 0; k < kSteps; ++k) v[k] = -((float)NMAX + 0.1f * (float)(k < 9 ? k - 9 : k - 8));
+  }
+};
+static __constant__ const QxNums<4> kQxQ3 = QxNums<4>();
+static __constant__ const QxNums<32> kQxQ6 = QxNums<32>();
+
+// Result of fit_signed: the scale and the inverse scale whose codes are the best
+// (signed_final_codes forms them), plus what the requantization's float form needs.
+struct SignedFit {
+  float scale, inv;
+  float amax;  // largest |x| (numpy's rules; meaningful to the float forms when fin)
+  bool dead, fin;
+};
+
+// clip(nearest_int(inv * x), -nmax, nmax - 1) + nmax of the best candidate (nmax for a
+// dead block).
 template <int N>
-__device__ __forceinline__ float fit_signed(const float (&x)[N], const float (&w)[N], int nmax,
-                                            int (&L)[N]) {
+__device__ __forceinline__ void signed_final_codes(const float (&x)[N], const SignedFit& f, int nmax,
+                                                   int (&L)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    L[i] = (f.dead ? 0 : clampi(rint_magic(f.inv * x[i]), -nmax, nmax - 1)) + nmax;
+}
+
+// Codes of one candidate, clip(nearest_int(inv * x), -nmax, nmax - 1), as floats. FAST as in
+// affine_codes. A negative product that rounds to zero gives -0 there and +0 in the integer
+// form: every sum the codes enter ends as 0.0f + s, so no result depends on it.
+template <int N, int NMAX, bool FAST>
+__device__ __forceinline__ void signed_codes(const float (&x)[N], float inv, float (&lf)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float v = inv * x[i];
+    if constexpr (FAST)
+      lf[i] = __builtin_rintf(__builtin_amdgcn_fmed3f(v, (float)-NMAX, (float)(NMAX - 1)));
+    else
+      lf[i] = (float)clampi(rint_magic(v), -NMAX, NMAX - 1);
+  }
+}
+
+// Symmetric signed fit x ~ scale * L, L in [-nmax, nmax-1]; weights w (pass x*x for the
+// unweighted path). VALU-bound: 19 candidates of N codes, three products a code and two
+// pairwise sums. The search keeps the best candidate's inverse scale instead of its codes
+// (the encoders requantize every sub-block whose grid step is non-zero, so the codes are
+// formed only where it is zero), and forms codes by med3 + rint: with every x finite,
+// |inv_c * x| <= (nmax + 0.9) |x| / amax (1 + 2^-23), far inside the range where that equals
+// the integer form, so the choice is made once, for the whole wave. The candidates share the
+// divisor sext. [151936, 1024] in plain Q6_K: 1043 -> 720 us with the packing by words
+// (147 VALU instructions a candidate instead of 231; 97 registers instead of 123).
+template <int N, class NUMS>
+__device__ __forceinline__ SignedFit fit_signed(const float (&x)[N], const float (&w)[N],
+                                                const NUMS& nums) {
+  constexpr int nmax = NUMS::kNmax;
   float amax = fabsf(x[0]), sext = x[0];
+  bool fin = isfinite(x[0]);
 #pragma unroll
   for (int i = 1; i < N; ++i) {
     float a = fabsf(x[i]);
+    fin = fin && isfinite(x[i]);
     if (a > amax) {
       amax = a;
       sext = x[i];
@@ -213,46 +270,65 @@ __device__ __forceinline__ float fit_signed(const float (&x)[N], const float (&w
 #pragma unroll
   for (int i = 0; i < N; ++i) wx[i] = w[i] * x[i];
 
-  float inv = -(float)nmax / sext;
-  float p[N], q[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    L[i] = clampi(rint_magic(inv * x[i]), -nmax, nmax - 1);
-    float lf = (float)L[i];
-    p[i] = wx[i] * lf;
-    q[i] = (w[i] * lf) * lf;
-  }
-  float slx = psum<N>(p), sl2 = psum<N>(q);
-  float scale = sl2 != 0.0f ? slx / sl2 : 0.0f;
-  float best = scale * slx;
-  for (int s = -9; s <= 9; ++s) {
-    if (s == 0) continue;
-    float inv_c = -((float)nmax + 0.1f * (float)s) / sext;
-    int Lc[N];
+  const bool fast = __all(fin), box = __all(div_box(sext));
+  const float y = div_recip(sext);
+  float lf[N], slx, sl2;
+  // sum_lx and sum_l2 of one candidate's codes, accumulated in psum's order as the products
+  // are formed
+  const auto sums = [&](float inv) {
+    if (fast)
+      signed_codes<N, nmax, true>(x, inv, lf);
+    else
+      signed_codes<N, nmax, false>(x, inv, lf);
+    float p8[8], q8[8];
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      Lc[i] = clampi(rint_magic(inv_c * x[i]), -nmax, nmax - 1);
-      float lf = (float)Lc[i];
-      p[i] = wx[i] * lf;
-      q[i] = (w[i] * lf) * lf;
+      const float p = wx[i] * lf[i], q = (w[i] * lf[i]) * lf[i];
+      p8[i % 8] = i < 8 ? p : p8[i % 8] + p;
+      q8[i % 8] = i < 8 ? q : q8[i % 8] + q;
     }
-    float slx_c = psum<N>(p), sl2_c = psum<N>(q);
-    if (sl2_c > 0.0f && slx_c * slx_c > best * sl2_c && !dead) {
-      float s_c = slx_c / sl2_c;
-#pragma unroll
-      for (int i = 0; i < N; ++i) L[i] = Lc[i];
+    slx = psum_tree(p8);
+    sl2 = psum_tree(q8);
+  };
+  float best_inv = -(float)nmax / sext;
+  sums(best_inv);
+  float scale = sl2 != 0.0f ? slx / sl2 : 0.0f;
+  float best = scale * slx;
+  for (int s = 0; s < NUMS::kSteps; ++s) {
+    const float num = nums.v[s];  // in div_box
+    const float inv_c = box ? div_by(num, sext, y) : num / sext;
+    sums(inv_c);
+    if (sl2 > 0.0f && slx * slx > best * sl2 && !dead) {
+      const float s_c = slx / sl2;
+      best_inv = inv_c;
       scale = s_c;
-      best = s_c * slx_c;
+      best = s_c * slx;
     }
   }
-  if (dead) {
-    scale = 0.0f;
+  return SignedFit{dead ? 0.0f : scale, best_inv, amax, dead, fin};
+}
+
+// clip(nearest_int(x / step), -nmax, nmax - 1) + nmax for a non-zero step: the encoders'
+// requantization on the committed grid. With x finite, |step| in [2^-24, 2^40], amax <= 2^40
+// and amax <= 2^21 |step| on every lane of the wave, the quotients share the reciprocal of
+// step (div_by) and round by med3 + rint. An |x| below div_box (2^-40) needs no test there:
+// its quotient is below 2^-16 whatever its last bits, so its code is 0 either way. A step
+// is an fp16 value times an integer, so it is below 2^-24 only when it is zero.
+template <int N>
+__device__ __forceinline__ void signed_requant(const float (&x)[N], const SignedFit& f, float step,
+                                               int nmax, int (&L)[N]) {
+  const float m = fabsf(step);
+  const bool ok = f.fin && f.amax <= 0x1p40f && m <= 0x1p40f && f.amax <= 0x1p21f * m;
+  if (__all(ok)) {
+    const float y = div_recip(step);
 #pragma unroll
-    for (int i = 0; i < N; ++i) L[i] = 0;
+    for (int i = 0; i < N; ++i)
+      L[i] = (int)__builtin_rintf(__builtin_amdgcn_fmed3f(div_by(x[i], step, y), (float)-nmax,
+                                                           (float)(nmax - 1))) + nmax;
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) L[i] = clampi(rint_magic(x[i] / step), -nmax, nmax - 1) + nmax;
   }
-#pragma unroll
-  for (int i = 0; i < N; ++i) L[i] += nmax;
-  return scale;
 }
 
 // Coordinate descent on fixed-grid codes, elements visited in order, at most 5

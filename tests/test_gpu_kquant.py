@@ -55,6 +55,28 @@ def test_matches_oracle_seeded(kq, tt, weighted):
         assert np.array_equal(rec.view(np.uint32), K.DEQUANTIZE[tt](want, n).view(np.uint32))
 
 
+@pytest.mark.parametrize("tt", ["Q3_K", "Q6_K"])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_signed_fits_over_the_float_range(kq, tt, weighted):
+    """The signed searches' float codes and shared divisors against the oracle where their
+    conditions change: sub-blocks around 1e-15 (the dead bound), 2^-40 (an end of the shared
+    divisor's range) and the fp16 scale's underflow, and tiny sub-blocks in superblocks whose
+    step is set by large ones (quotients past the float form's range take the integer one)."""
+    rng = np.random.default_rng(91)
+    x = rng.standard_normal((24, 512)) * 10.0 ** rng.uniform(-18, 4, (24, 32)).repeat(16, axis=1)
+    for r, m in enumerate((1e-15, 0.9e-15, 2.0 ** -40, 2.0 ** -39, 6e-8, 3e-5)):
+        x[r, :256] = rng.standard_normal(256) * m
+    x[6, 16:32] = 1e-6                 # one tiny sub-block in an ordinary superblock
+    x[6, :16] = rng.standard_normal(16)
+    x = x.astype(np.float32)
+    qw = (np.abs(rng.standard_normal(512)) + 0.1).astype(np.float32) if weighted else None
+    with np.errstate(all="ignore"):
+        want = K.QUANTIZE[tt](x, qw)
+    got = kq.QUANTIZE[tt](x, qw)
+    bad = np.nonzero((got != want).any(1))[0]
+    assert bad.size == 0, f"rows {bad} differ"
+
+
 @pytest.mark.parametrize("tt", CODEC_TYPES)
 def test_empty_tensors_behave_like_the_reference(kq, tt):
     """Zero rows: the reference's encoders fail in their final reshape(nrow, -1) with
