@@ -4,8 +4,8 @@
 //     sum_c w[c] * sum_r (roundtrip(x[rows][:, perm])[r, c] - x[rows][r, perm[c]])^2
 // with w = wvec[perm], qw[perm] or 1, evaluated for many tensors in one pass:
 //   gather   x rows (a sorted sample) and permuted columns, f16 or f32 -> f32
-//   encode   the container codec bodies of kq_blocks.h, one launch per type group
-//   decode   the same decoders as cp_kq_dequantize
+//   encode   the container codec bodies of kq_blocks.h, one launch per type group, which
+//            write the decoded weights (Q8_0: bytes, then its decoder)
 //   colsum   per column, the float64 squared errors added row after row -- the
 //            order of numpy's d2.sum(0) over a C-contiguous array, so the result is
 //            bit-identical
@@ -29,6 +29,7 @@ namespace cp {
 // and forces the loads ahead of it to drain).
 typedef const float __attribute__((address_space(1)))* GF32;
 typedef const uint16_t __attribute__((address_space(1)))* GU16;
+typedef const int32_t __attribute__((address_space(1)))* GI32;
 
 struct ErrDev {
   const void* x;
@@ -38,24 +39,91 @@ struct ErrDev {
   const double* wvec;
   float* xs;       // [R, n] gathered targets
   float* qwp;      // [n] qw[perm] (or null)
-  uint8_t* raw;    // [R, n / block_weights * block_bytes]
+  uint8_t* raw;    // Q8_0's bytes [R, n / 32 * 34] (the k-quants leave none)
   float* recon;    // [R, n]
   double* colerr;  // [n]
   int* bad;        // set when an index is out of range
   int64_t nrow_src;
   int R, n, ttype, x_f16;
   int slot;  // the caller's index of this tensor (its result slot)
+  int gfirst;  // first workgroup of the gather that works on this tensor
+  int by_rows; // table index of the tensor with the k-th most rows, k this entry's index
 };
 
 // --------------------------------------------------------------- gather
-// Four consecutive columns of one gathered row per thread (n % 32 == 0, so the
-// four never straddle rows). Negative indices count from the end, as numpy's do;
-// indices still out of range read element 0 and flag the tensor, whose result
-// becomes NaN.
-__global__ __launch_bounds__(256) void err_gather_kernel(const ErrDev* __restrict__ tab) {
-  const ErrDev& T = tab[blockIdx.y];
+// Workgroups take tiles of kGatherRows rows x 1024 columns, tensor by tensor (gfirst), so a
+// call of one large and many small tensors launches no idle ones. A thread keeps its four
+// consecutive columns' indices in registers over the tile's rows, so an entry costs its
+// gathered load and a quarter of a 16-byte store. (One thread per four entries of a
+// (largest tensor, tensors) grid, reading and checking its indices for every row, took
+// 238 us for 29 tensors of 1 M - 16.8 M entries; this takes 138, 3.5 TB/s of f16 in and f32 out.) Negative indices count from
+// the end, as numpy's do; indices still out of range read element 0 and flag the tensor, whose
+// result becomes NaN.
+constexpr int kGatherRows = 32, kGatherCols = 1024;
+
+template <bool F16>
+__device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int j) {
   const int n = T.n;
-  if (blockIdx.x == 0 && T.qwp) {
+  const GU16 x16 = (GU16)T.x;
+  const GF32 x32 = (GF32)T.x;
+  const GI32 perm = (GI32)T.perm, rows = (GI32)T.rows;
+  bool bad = false;
+  int c[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    c[q] = perm ? perm[j + q] : j + q;
+    c[q] = c[q] < 0 ? c[q] + n : c[q];
+    if (c[q] < 0 || c[q] >= n) {
+      bad = true;
+      c[q] = 0;
+    }
+  }
+  const auto row_of = [&](int i) {
+    int64_t src = rows ? rows[i] : i;
+    src = src < 0 ? src + T.nrow_src : src;
+    if (src < 0 || src >= T.nrow_src) {
+      bad = true;
+      src = 0;
+    }
+    return src * n;
+  };
+  float4* out = reinterpret_cast<float4*>(T.xs + j);
+  constexpr int U = 8;  // rows in flight
+  int i = i0;
+  for (; i + U <= i1; i += U) {
+    float v[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t o = row_of(i + u);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[u][q] = F16 ? half_value(x16[o + c[q]]) : x32[o + c[q]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      out[(int64_t)(i + u) * (n / 4)] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+  }
+  for (; i < i1; ++i) {
+    const int64_t o = row_of(i);
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = F16 ? half_value(x16[o + c[q]]) : x32[o + c[q]];
+    out[(int64_t)i * (n / 4)] = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  if (bad) *T.bad = 1;
+}
+
+__global__ __launch_bounds__(256) void err_gather_kernel(const ErrDev* __restrict__ tab, int count) {
+  int lo = 0, hi = count - 1;  // the last tensor with gfirst <= blockIdx.x
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (tab[mid].gfirst <= (int)blockIdx.x)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  const ErrDev& T = tab[lo];
+  const int blk = (int)blockIdx.x - T.gfirst, n = T.n;
+  if (blk == 0 && T.qwp) {
     for (int j = threadIdx.x; j < n; j += 256) {
       int c = T.perm ? T.perm[j] : j;
       c = c < 0 ? c + n : c;  // numpy's negative indices
@@ -66,28 +134,20 @@ __global__ __launch_bounds__(256) void err_gather_kernel(const ErrDev* __restric
       T.qwp[j] = T.qw[c];
     }
   }
-  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (e >= (int64_t)T.R * n) return;
-  const int i = (int)(e / n), j = (int)(e - (int64_t)i * n);
-  int64_t src = T.rows ? T.rows[i] : i;
-  src = src < 0 ? src + T.nrow_src : src;
-  bool bad = src < 0 || src >= T.nrow_src;
-  src = bad ? 0 : src;
-  float v[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    int c = T.perm ? T.perm[j + k] : j + k;
-    c = c < 0 ? c + n : c;
-    if (c < 0 || c >= n) {
-      bad = true;
-      c = 0;
-    }
-    const int64_t o = src * n + c;
-    v[k] = T.x_f16 ? half_value(reinterpret_cast<const uint16_t*>(T.x)[o])
-                   : reinterpret_cast<const float*>(T.x)[o];
-  }
-  if (bad) *T.bad = 1;
-  reinterpret_cast<float4*>(T.xs)[e >> 2] = make_float4(v[0], v[1], v[2], v[3]);
+  const int ct = (n + kGatherCols - 1) / kGatherCols, rt = blk / ct;
+  const int j = (blk - rt * ct) * kGatherCols + 4 * (int)threadIdx.x;
+  if (j >= n) return;  // n % 32 == 0: the four columns exist together
+  const int64_t i0 = (int64_t)rt * kGatherRows;
+  const int i1 = (int)(T.R - i0 < kGatherRows ? T.R : i0 + kGatherRows);
+  if (T.x_f16)
+    gather_tile<true>(T, (int)i0, i1, j);
+  else
+    gather_tile<false>(T, (int)i0, i1, j);
+}
+
+// Workgroups of one tensor's gather.
+static int64_t gather_tiles(int64_t R, int64_t n) {
+  return ((R + kGatherRows - 1) / kGatherRows) * ((n + kGatherCols - 1) / kGatherCols);
 }
 
 // --------------------------------------------------------------- codec
@@ -104,27 +164,17 @@ __global__ __launch_bounds__(256) void err_encode_kernel(const ErrDev* __restric
     const int64_t NB = w / 256;
     const int64_t blocks = ((NB + S - 1) / S + kWavesPerBlock - 1) / kWavesPerBlock;
     if ((int64_t)blockIdx.x >= blocks) return;
-    kq_encode_block<TT, IMAT>(T.xs, T.qwp, NB, T.n / 256, T.raw, blockIdx.x);
+    kq_encode_block<TT, IMAT, KqOut::kRecon>(T.xs, T.qwp, NB, T.n / 256, nullptr, blockIdx.x, T.recon);
   }
 }
 
-// Q8_0: one thread per 4 weights; k-quants: 16 superblocks per workgroup
-// (kq_decode_block).
-template <int TT>
-__global__ __launch_bounds__(256) void err_decode_kernel(const ErrDev* __restrict__ tab) {
+// Q8_0: one thread per 4 weights.
+__global__ __launch_bounds__(256) void err_decode_q8_kernel(const ErrDev* __restrict__ tab) {
   const ErrDev& T = tab[blockIdx.y];
-  const int64_t w = (int64_t)T.R * T.n;
-  if constexpr (TT == CP_Q8_0) {
-    q8_decode_thread(T.raw, w / 32, T.recon, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-  } else {
-    __shared__ __align__(16) KqDecodeLds<TT> lds;
-    kq_decode_block<TT>(T.raw, w / 256, T.recon, blockIdx.x, lds);
-  }
+  q8_decode_thread(T.raw, (int64_t)T.R * T.n / 32, T.recon, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // --------------------------------------------------------------- column sums
-// One lane per column: colerr[c] = (((0 + d2[0,c]) + d2[1,c]) + ...), d2 the
-// float64 square of the float64 difference, loads pipelined by chain_rows.
 // The sequential chain of one column over rows [r0, r1), loads running one block
 // of B rows ahead of the adds. The block after next is always loaded (clamped to
 // the last full block), so no branch sits between a load and its use and the
@@ -157,123 +207,158 @@ __device__ __forceinline__ void chain_rows(int64_t r0, int64_t r1, const Ld& ld,
   }
 }
 
-__global__ __launch_bounds__(64) void err_colsum_kernel(const ErrDev* __restrict__ tab) {
-  const ErrDev& T = tab[blockIdx.y];
-  const int c = blockIdx.x * 64 + threadIdx.x;
+// colerr[c] = (((0 + d2[0,c]) + d2[1,c]) + ...), d2 the float64 square of the float64
+// difference. The order makes each column one chain of R additions, so a column's time is
+// that chain or the delivery of its values, whichever is longer. A workgroup takes 32 columns
+// (128-byte row segments): seven waves load four tiles ahead and put the squares, which are off
+// the chain, into a double-buffered LDS tile; the eighth only adds, one lane per column,
+// reading 16 rows ahead of the adds. One wave doing it all for 64 columns, its loads one
+// 16-row block ahead, took 741 us for 29 tensors (79.7 M entries, one of 16384 rows) where this
+// takes 228, the tensors with the most rows first (269 in table order): 2.8 TB/s.
+constexpr int kSumCols = 32, kSumWaves = 8, kSumPer = 8, kSumAhead = 4;
+constexpr int kSumRows = (kSumWaves - 1) * 2 * kSumPer;  // 112 rows per tile
+
+__global__ __launch_bounds__(64 * kSumWaves) void err_colsum_kernel(const ErrDev* __restrict__ tab) {
+  const ErrDev& T = tab[tab[blockIdx.y].by_rows];  // longest chains first
   const int64_t n = T.n;
-  if (c >= n) return;
-  const GF32 xs = (GF32)T.xs;
-  const GF32 rc = (GF32)T.recon;
-  double acc = 0.0;
-  chain_rows<16, float2>(
-      0, T.R, [&](int64_t r) { return make_float2((xs + r * n)[c], (rc + r * n)[c]); },
-      [&](float2 v) {
-        const double d = (double)v.y - (double)v.x;
-        acc = acc + d * d;
-      });
-  T.colerr[c] = acc;
+  const int c0 = (int)blockIdx.x * kSumCols;
+  if (c0 >= n) return;  // n % 32 == 0: all 32 columns exist
+  __shared__ double d2[2][kSumRows][kSumCols];
+  const int R = T.R, tiles = (R + kSumRows - 1) / kSumRows;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), c = (int)threadIdx.x & 31;
+  if (wv < kSumWaves - 1) {
+    const GF32 xs = (GF32)T.xs + c0 + c;
+    const GF32 rc = (GF32)T.recon + c0 + c;
+    const int g = ((int)threadIdx.x >> 5) * kSumPer;  // this thread's first row of a tile
+    float2 v[kSumAhead][kSumPer];
+    auto fill = [&](float2 (&d)[kSumPer], int tile) {
+#pragma unroll
+      for (int i = 0; i < kSumPer; ++i) {  // past the last row: that row again, never added
+        const int64_t r = (int64_t)tile * kSumRows + g + i, rr = r < R ? r : R - 1;
+        d[i] = make_float2(xs[rr * n], rc[rr * n]);
+      }
+    };
+#pragma unroll
+    for (int a = 0; a < kSumAhead; ++a) fill(v[a], a);
+    for (int k = 0; k < tiles; k += kSumAhead) {  // every wave passes the same ``tiles`` barriers
+#pragma unroll
+      for (int a = 0; a < kSumAhead; ++a) {
+        if (k + a >= tiles) break;
+#pragma unroll
+        for (int i = 0; i < kSumPer; ++i) {
+          const double d = (double)v[a][i].y - (double)v[a][i].x;
+          d2[a & 1][g + i][c] = d * d;
+        }
+        __syncthreads();
+        fill(v[a], k + a + kSumAhead);
+      }
+    }
+  } else {
+    // tile k is whole after barrier k; its buffer is written again only after barrier k + 1,
+    // which this wave passes when it has added tile k
+    double acc = 0.0;
+    for (int k = 0; k < tiles; ++k) {
+      __syncthreads();
+      const double(*p)[kSumCols] = d2[k & 1];
+      const int rows = R - k * kSumRows < kSumRows ? R - k * kSumRows : kSumRows;
+      if (rows == kSumRows) {
+        double v[2][16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[0][i] = p[i][c];
+#pragma unroll
+        for (int q = 0; q < kSumRows / 16; ++q) {
+          if (q + 1 < kSumRows / 16) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[(q + 1) & 1][i] = p[16 * (q + 1) + i][c];
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc = acc + v[q & 1][i];
+        }
+      } else {
+        for (int r = 0; r < rows; ++r) acc = acc + p[r][c];
+      }
+    }
+    if (((int)threadIdx.x & 63) < kSumCols) T.colerr[c0 + c] = acc;
+  }
 }
 
 // --------------------------------------------------------------- pairwise sum
-// numpy's summation of a float64 array of n values v(i). It reduces in chunks
-// of 8192 values (its ufunc buffer size), adding the chunk sums left to right
-// onto +0.0. Inside a chunk the sum is pairwise: fewer than 8 values
-// sequentially from 0.0; up to 128 with eight strided accumulators,
-// ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)), then the remainder; longer runs split at
-// n/2 rounded down to a multiple of 8, the two halves summed recursively. The
-// recursion runs on an explicit stack (depth <= 32).
-template <class V>
-__device__ double pw_leaf(const V& v, int64_t lo, int64_t n) {
-  if (n < 8) {
-    double r = 0.0;
-    for (int64_t i = 0; i < n; ++i) r = r + v(lo + i);
-    return r;
-  }
-  double r[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = v(lo + j);
-  int64_t i = 8;
-  for (; i < n - (n % 8); i += 8) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) r[j] = r[j] + v(lo + i + j);
-  }
-  double s = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
-  for (; i < n; ++i) s = s + v(lo + i);
-  return s;
-}
+// numpy's summation of a contiguous float64 array of n values v(i), n % 8 == 0. It reduces in
+// chunks of 8192 values (its ufunc buffer size), adding the chunk sums left to right onto
+// +0.0. Inside a chunk the sum is pairwise: up to 128 values with eight strided accumulators,
+// ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)); longer runs split at n/2 rounded down to a multiple of
+// 8, the two halves summed recursively. (With n % 8 == 0 every run is a multiple of 8, so no
+// run has a remainder.) One workgroup: the chunk's split tree is laid out as a heap (node i,
+// halves 2i and 2i + 1; m splits into at most m/2 + 8, so 8192 values end at level 7), the
+// leaves summed in parallel by 8 lanes each, and the halves added level by level. One lane
+// walking the tree took 167 us for 29 tensors up to n = 3072; this takes 13.
+constexpr int kNpChunk = 8192, kTreeNodes = 256;
 
 template <class V>
-__device__ double pw_tree(const V& v, int64_t lo0, int64_t n) {
-  struct Frame {
-    int64_t lo, n;
-    double left;
-    int right;
-  };
-  Frame st[32];
-  int sp = 0;
-  st[0] = Frame{lo0, n, 0.0, 0};
-  for (;;) {
-    Frame& f = st[sp];
-    if (f.n <= 128) {
-      double val = pw_leaf(v, f.lo, f.n);
-      for (;;) {  // hand the value to the parents
-        if (--sp < 0) return val;
-        Frame& p = st[sp];
-        if (!p.right) {
-          p.left = val;
-          p.right = 1;
-          int64_t n2 = p.n / 2;
-          n2 -= n2 % 8;
-          st[sp + 1] = Frame{p.lo + n2, p.n - n2, 0.0, 0};
-          ++sp;
-          break;
-        }
-        val = p.left + val;
-      }
-    } else {
-      int64_t n2 = f.n / 2;
-      n2 -= n2 % 8;
-      f.right = 0;
-      st[sp + 1] = Frame{f.lo, n2, 0.0, 0};
-      ++sp;
-    }
-  }
-}
-
-constexpr int64_t kNpChunk = 8192;
-
-template <class V>
-__device__ double pw_sum(const V& v, int64_t n) {
+__device__ double pw_sum_block(const V& v, int64_t n, int2* node, double* val) {
   double s = 0.0;
-  for (int64_t c0 = 0; c0 < n; c0 += kNpChunk) s = s + pw_tree(v, c0, n - c0 < kNpChunk ? n - c0 : kNpChunk);
+  const int t = (int)threadIdx.x;
+  for (int64_t c0 = 0; c0 < n; c0 += kNpChunk) {
+    __syncthreads();
+    if (t == 0) node[1] = make_int2(0, (int)(n - c0 < kNpChunk ? n - c0 : kNpChunk));
+    for (int first = 1; first < kTreeNodes / 2; first *= 2) {
+      __syncthreads();
+      if (t < first) {
+        const int2 p = node[first + t];
+        const int h = p.y > 128 ? p.y / 2 / 8 * 8 : 0;  // 0: a leaf, or absent (y == 0)
+        node[2 * (first + t)] = make_int2(p.x, h);
+        node[2 * (first + t) + 1] = make_int2(p.x + h, h ? p.y - h : 0);
+      }
+    }
+    __syncthreads();
+    for (int i = 1 + t / 8; i < kTreeNodes; i += 32) {
+      const int2 p = node[i];
+      const bool leaf = p.y > 0 && p.y <= 128;
+      double r = 0.0;
+      if (leaf) {
+        const int64_t o = c0 + p.x + t % 8;
+        r = v(o);
+        for (int k = 8; k < p.y; k += 8) r = r + v(o + k);
+      }
+      r = r + __shfl_xor(r, 1);
+      r = r + __shfl_xor(r, 2);
+      r = r + __shfl_xor(r, 4);
+      if (leaf && t % 8 == 0) val[i] = r;
+    }
+    for (int first = kTreeNodes / 4; first >= 1; first /= 2) {
+      __syncthreads();
+      if (t < first && node[first + t].y > 128) val[first + t] = val[2 * (first + t)] + val[2 * (first + t) + 1];
+    }
+    __syncthreads();
+    s = s + val[1];
+  }
   return s;
 }
 
-__global__ __launch_bounds__(64) void err_final_kernel(const ErrDev* __restrict__ tab,
-                                                       double* __restrict__ out) {
-  if (threadIdx.x != 0) return;
+__global__ __launch_bounds__(256) void err_final_kernel(const ErrDev* __restrict__ tab,
+                                                        double* __restrict__ out) {
+  __shared__ int2 node[kTreeNodes];
+  __shared__ double val[kTreeNodes];
   const ErrDev& T = tab[blockIdx.x];
-  if (*T.bad) {
-    out[T.slot] = __builtin_nan("");
-    return;
-  }
-  const double* ce = T.colerr;
   double s;
-  if (T.wvec) {
+  const double* ce = T.colerr;
+  if (*T.bad) {
+    s = __builtin_nan("");
+  } else if (T.wvec) {
     const int32_t* perm = T.perm;
     const double* wv = T.wvec;
     const int64_t n = T.n;
-    s = pw_sum([=](int64_t i) {
+    s = pw_sum_block([=](int64_t i) {
       const int64_t c = perm ? perm[i] : i;
       return ce[i] * wv[c < 0 ? c + n : c];
-    }, T.n);
+    }, T.n, node, val);
   } else if (T.qwp) {
     const float* q = T.qwp;
-    s = pw_sum([=](int64_t i) { return ce[i] * (double)q[i]; }, T.n);
+    s = pw_sum_block([=](int64_t i) { return ce[i] * (double)q[i]; }, T.n, node, val);
   } else {
-    s = pw_sum([=](int64_t i) { return ce[i]; }, T.n);
+    s = pw_sum_block([=](int64_t i) { return ce[i]; }, T.n, node, val);
   }
-  out[T.slot] = s;
+  if (threadIdx.x == 0) out[T.slot] = s;
 }
 
 __global__ void err_clear_kernel(int* __restrict__ bad, int count) {
@@ -347,7 +432,7 @@ static ErrLayout err_layout(const cp_err_tensor& t, size_t o) {
   ErrLayout L;
   L.xs = o; o += a256((size_t)R * t.n * 4);
   L.qwp = o; o += a256((size_t)t.n * 4);
-  L.raw = o; o += a256((size_t)R * (t.n / g.block_weights) * g.block_bytes);
+  L.raw = o; o += t.ttype == CP_Q8_0 ? a256((size_t)R * (t.n / g.block_weights) * g.block_bytes) : 0;
   L.recon = o; o += a256((size_t)R * t.n * 4);
   L.colerr = o; o += a256((size_t)t.n * 8);
   L.end = o;
@@ -364,7 +449,7 @@ size_t err_ws_bytes(const cp_err_tensor* ts, int count) {
   return o;
 }
 
-constexpr int kErrPerStore = 32;
+constexpr int kErrPerStore = 31;
 struct ErrBatch {
   ErrDev t[kErrPerStore];
 };
@@ -406,33 +491,16 @@ static void launch_err_encode(const ErrDev* tab, const ErrGroup& g, hipStream_t 
     err_encode_kernel<TT, false><<<grid, 256, 0, st>>>(tab + g.first);
 }
 
-template <int TT>
-static void launch_err_decode(const ErrDev* tab, const ErrGroup& g, hipStream_t st) {
-  // Q8_0: one thread per 4 weights; k-quants: 16 superblocks per workgroup
-  const int64_t blocks = TT == CP_Q8_0 ? (g.max_w / 4 + 255) / 256
-                                       : (g.max_w / 256 + 4 * kDecSb - 1) / (4 * kDecSb);
-  err_decode_kernel<TT><<<dim3((unsigned)blocks, (unsigned)g.count), 256, 0, st>>>(tab + g.first);
-}
-
-template <template <int> class L>
-static void for_group_type(const ErrDev* tab, const ErrGroup& g, hipStream_t st) {
+static void launch_err_group(const ErrDev* tab, const ErrGroup& g, hipStream_t st) {
   switch (g.ttype) {
-    case CP_Q8_0: L<CP_Q8_0>::run(tab, g, st); break;
-    case CP_Q2_K: L<CP_Q2_K>::run(tab, g, st); break;
-    case CP_Q3_K: L<CP_Q3_K>::run(tab, g, st); break;
-    case CP_Q4_K: L<CP_Q4_K>::run(tab, g, st); break;
-    case CP_Q5_K: L<CP_Q5_K>::run(tab, g, st); break;
-    default: L<CP_Q6_K>::run(tab, g, st); break;
+    case CP_Q8_0: launch_err_encode<CP_Q8_0>(tab, g, st); break;
+    case CP_Q2_K: launch_err_encode<CP_Q2_K>(tab, g, st); break;
+    case CP_Q3_K: launch_err_encode<CP_Q3_K>(tab, g, st); break;
+    case CP_Q4_K: launch_err_encode<CP_Q4_K>(tab, g, st); break;
+    case CP_Q5_K: launch_err_encode<CP_Q5_K>(tab, g, st); break;
+    default: launch_err_encode<CP_Q6_K>(tab, g, st); break;
   }
 }
-template <int TT>
-struct EncodeL {
-  static void run(const ErrDev* t, const ErrGroup& g, hipStream_t st) { launch_err_encode<TT>(t, g, st); }
-};
-template <int TT>
-struct DecodeL {
-  static void run(const ErrDev* t, const ErrGroup& g, hipStream_t st) { launch_err_decode<TT>(t, g, st); }
-};
 
 int err_batch(const cp_err_tensor* ts, int count, void* ws, size_t ws_bytes, double* out,
               hipStream_t st) {
@@ -464,7 +532,6 @@ int err_batch(const cp_err_tensor* ts, int count, void* ws, size_t ws_bytes, dou
   std::vector<ErrDev> devs(count);
   size_t o = err_tables_bytes(count);
   int max_n = 0;
-  int64_t max_w = 0;
   for (int i = 0; i < count; ++i) {
     const cp_err_tensor& t = ts[i];
     const ErrLayout L = err_layout(t, o);
@@ -473,9 +540,8 @@ int err_batch(const cp_err_tensor* ts, int count, void* ws, size_t ws_bytes, dou
     devs[i] = ErrDev{t.x, t.rows, t.perm, t.qw, t.wvec,
                      (float*)(base + L.xs), t.qw ? (float*)(base + L.qwp) : nullptr,
                      (uint8_t*)(base + L.raw), (float*)(base + L.recon), (double*)(base + L.colerr),
-                     bad + i, t.nrow, R, (int)t.n, t.ttype, t.x_dtype, i};
+                     bad + i, t.nrow, R, (int)t.n, t.ttype, t.x_dtype, i, 0, 0};
     max_n = (int)t.n > max_n ? (int)t.n : max_n;
-    max_w = (int64_t)R * t.n > max_w ? (int64_t)R * t.n : max_w;
   }
   // table ordered by (type, importance) so each codec group is one run of rows
   std::vector<int> order(count);
@@ -485,7 +551,17 @@ int err_batch(const cp_err_tensor* ts, int count, void* ws, size_t ws_bytes, dou
     return (ts[a].qw != nullptr) < (ts[b].qw != nullptr);
   });
   std::vector<ErrDev> sorted(count);
-  for (int k = 0; k < count; ++k) sorted[k] = devs[order[k]];
+  int64_t gather_blocks = 0;
+  for (int k = 0; k < count; ++k) {
+    sorted[k] = devs[order[k]];
+    sorted[k].gfirst = (int)gather_blocks;
+    gather_blocks += gather_tiles(sorted[k].R, sorted[k].n);
+    if (gather_blocks > 0x7FFFFFFF) return set_error(CP_ERR_SHAPE, "too many weights in one call");
+  }
+  std::vector<int> by_rows(count);
+  for (int k = 0; k < count; ++k) by_rows[k] = k;
+  std::stable_sort(by_rows.begin(), by_rows.end(), [&](int a, int b) { return sorted[a].R > sorted[b].R; });
+  for (int k = 0; k < count; ++k) sorted[k].by_rows = by_rows[k];
   std::vector<ErrGroup> groups;
   for (int k = 0; k < count; ++k) {
     const ErrDev& d = sorted[k];
@@ -505,19 +581,23 @@ int err_batch(const cp_err_tensor* ts, int count, void* ws, size_t ws_bytes, dou
   }
   CP_PHASE_MARK(g_err_clock, -1);
   err_clear_kernel<<<(count + 255) / 256, 256, 0, st>>>(bad, count);
-  err_gather_kernel<<<dim3((unsigned)((max_w / 4 + 255) / 256), (unsigned)count), 256, 0, st>>>(dtab);
+  err_gather_kernel<<<(unsigned)gather_blocks, 256, 0, st>>>(dtab, count);
   CP_LAUNCHED("objective gather");
   CP_PHASE_MARK(g_err_clock, 0);
-  for (const ErrGroup& g : groups) for_group_type<EncodeL>(dtab, g, st);
+  for (const ErrGroup& g : groups) launch_err_group(dtab, g, st);
   CP_LAUNCHED("objective encode");
   CP_PHASE_MARK(g_err_clock, 1);
-  for (const ErrGroup& g : groups) for_group_type<DecodeL>(dtab, g, st);
+  for (const ErrGroup& g : groups)
+    if (g.ttype == CP_Q8_0)
+      err_decode_q8_kernel<<<dim3((unsigned)((g.max_w / 4 + 255) / 256), (unsigned)g.count), 256, 0, st>>>(
+          dtab + g.first);
   CP_LAUNCHED("objective decode");
   CP_PHASE_MARK(g_err_clock, 2);
-  err_colsum_kernel<<<dim3((unsigned)((max_n + 63) / 64), (unsigned)count), 64, 0, st>>>(dtab);
+  err_colsum_kernel<<<dim3((unsigned)((max_n + kSumCols - 1) / kSumCols), (unsigned)count), 64 * kSumWaves, 0, st>>>(
+      dtab);
   CP_LAUNCHED("objective column sums");
   CP_PHASE_MARK(g_err_clock, 3);
-  err_final_kernel<<<count, 64, 0, st>>>(dtab, out);
+  err_final_kernel<<<count, 256, 0, st>>>(dtab, out);
   CP_LAUNCHED("objective total");
   CP_PHASE_MARK(g_err_clock, 4);
   return CP_OK;

@@ -51,6 +51,25 @@ def test_tensor_err_bit_identical(ob, tt, dtype):
         assert got == want, (k, got, want)
 
 
+@pytest.mark.parametrize("tt,nrow,n", [("Q8_0", 1, 32), ("Q8_0", 112, 96), ("Q4_K", 111, 256),
+                                       ("Q6_K", 113, 1280), ("Q3_K", 224, 512), ("Q2_K", 337, 256),
+                                       ("Q5_K", 9, 8448)])
+def test_tensor_err_at_tile_edges(ob, tt, nrow, n):
+    """Row counts around the column sums' 112-row tiles, gathers that end inside a run of 4096
+    entries and rows longer than one, and totals whose last chunk is short (8448 = 8192 + 256),
+    each alone and beside a larger tensor of another type."""
+    _say(f"tile edges {tt} [{nrow}, {n}]")
+    x = heavy_tailed(nrow, n, seed=nrow + n).astype(np.float16)
+    rng = np.random.default_rng(n)
+    qw, perm = (np.abs(rng.standard_normal(n)) + 0.05).astype(F32), rng.permutation(n)
+    want = Po.tensor_err(x, tt, qw, perm=perm)
+    assert ob.tensor_err(x, tt, qw, perm=perm) == want
+    other = heavy_tailed(150, 768, seed=3)
+    many = ob.tensor_err_many([dict(x=other, ttype="Q6_K", qw=None),
+                               dict(x=x, ttype=tt, qw=qw, perm=perm)])
+    assert many == [Po.tensor_err(other, "Q6_K", None), want]
+
+
 def _one_tree(v):
     """Pairwise sum of v as one tree (numpy's order only up to 8192 values)."""
     n = len(v)
