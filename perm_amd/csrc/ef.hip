@@ -1010,7 +1010,8 @@ __global__ __launch_bounds__(256) void ef_transpose_kernel(const EfDev* __restri
 // from the original weights (first iteration) or the compensated targets.
 // At most 168 VGPRs, three waves per SIMD: the 32-value sub-block searches of Q4_K and
 // Q5_K (146-152 registers since their pairwise sums accumulate as the terms are formed)
-// held 171-179 before, two waves per SIMD.
+// held 171-179 before, two waves per SIMD. Only the scale fields leave: the sweep forms the
+// codes, and ef_pack_kernel writes every code byte once, after the last iteration.
 template <int TT, bool IMAT>
 __global__ __launch_bounds__(256, 3) void ef_commit_kernel(const EfDev* __restrict__ tab, int from_wcur) {
   const EfDev& t = tab[blockIdx.y];
@@ -1018,7 +1019,7 @@ __global__ __launch_bounds__(256, 3) void ef_commit_kernel(const EfDev* __restri
   const int64_t nsb = t.n / 256, NB = (int64_t)t.nrow * nsb;
   const int64_t blocks = ((NB + S - 1) / S + kWavesPerBlock - 1) / kWavesPerBlock;
   if ((int64_t)blockIdx.x >= blocks) return;
-  kq_encode_block<TT, IMAT>(from_wcur ? t.Wcur : t.x, t.qw, NB, nsb, t.raw, blockIdx.x);
+  kq_encode_block<TT, IMAT, KqOut::kFields>(from_wcur ? t.Wcur : t.x, t.qw, NB, nsb, t.raw, blockIdx.x);
 }
 
 // 16 superblocks per workgroup (kq_decode_block); a tensor without a reconstruction
@@ -1467,9 +1468,10 @@ int ef_encode_batch(const cp_ef_tensor* ts, int count, int n_iter, int mode, voi
     CP_LAUNCHED("EF sweep");
     CP_PHASE(2);
     const int64_t pack_units = (int64_t)((max_rows + kPackRows - 1) / kPackRows) * (max_n / 256);
-    ef_pack_kernel<<<dim3((unsigned)pack_units, (unsigned)count), 256, 0, st>>>(dtab);
     if (it + 1 < n_iter)
       ef_transpose_kernel<2><<<dim3(col_tiles, row_tiles, (unsigned)count), 256, 0, st>>>(dtab);
+    else
+      ef_pack_kernel<<<dim3((unsigned)pack_units, (unsigned)count), 256, 0, st>>>(dtab);
     CP_LAUNCHED("EF repack");
     CP_PHASE(3);
   }
