@@ -82,6 +82,8 @@ def last_sweep_kernel(lib):
     import ctypes
     rs, wv = (ctypes.c_int * 1)(), (ctypes.c_int * 1)()
     lib.cp_ef_last_sweep(ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(wv, ctypes.c_void_p))
+    if rs[0] == 4:
+        return f"ef_sweep_quad_kernel ({wv[0]} waves)"
     if wv[0] > 1:
         return f"ef_sweep_pipe_kernel<{rs[0]}, {wv[0]}>"
     return f"ef_sweep_rows_kernel<{rs[0]}>"
@@ -105,7 +107,7 @@ def measure_sweep_traffic(layers):
                           os.path.join(tmp, f"copy_{counter}"))
         if len(copy) != 1 or copy[0][1] <= 0:
             raise RuntimeError(f"copy calibration: {len(copy)} dispatches of the copy kernel")
-        sweep = _pmc_child(counter, "ef_sweep_(rows|pipe)", ["--workload", "sweep-pass",
+        sweep = _pmc_child(counter, "ef_sweep_(rows|pipe|quad)", ["--workload", "sweep-pass",
                                                              "--layers", str(layers)],
                            os.path.join(tmp, f"sweep_{counter}"))
         if len(sweep) != 6:

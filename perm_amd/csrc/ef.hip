@@ -778,6 +778,288 @@ __global__ __launch_bounds__(64 * W, 2) void ef_sweep_pipe_kernel(const SweepTas
   }
 }
 
+// ---------------------------------------------------------------- quad stripes
+// Exact mode for calls with few rows: stripes of four rows, W waves each. Such a call is
+// bound by the column chain of one stripe, not by its arithmetic: a 16-row stripe's wave
+// issues about 70 VALU instructions a column (the row's updates on 16 registers, both
+// divisions, the stores), 280 ns a column with one wave on its SIMD, and 1024 rows fill 64 of
+// the 256 CUs. Here a column costs its wave about 27, 1024 rows take every CU, and a sweep of
+// [1024, n] takes 95 us for n = 1024 (283 before), 233 for 2048 (609), 427 for 3072 (1068) and
+// 681 for 4096 (1642; the stripes then read U at 12.6 TB/s from L2, eight waves a CU applying
+// earlier blocks):
+//   - the row's 64 columns lie over 16 lanes (lane l: row l / 16, columns l % 16 + 16 k in
+//     register k), so a column updates at most four registers, and its error reaches the
+//     row's lanes through the DPP row broadcast of the multiply that uses it;
+//   - every lane quantizes its own column's value against its own grid step (only the
+//     owner's result is used), so grid steps and their reciprocals stay in registers for
+//     16 columns, and the diagonal tile is in registers, loaded while earlier blocks are
+//     applied;
+//   - both divisions share reciprocals formed off the chain (div_recip; quad_div is div_by);
+//     the operand ranges that needs are checked with the column and a quarter block that
+//     fails is swept again by the general expressions from its saved targets;
+//   - errors go to the stripe's other waves through LDS in quarter blocks, so only the last
+//     quarter's updates separate two blocks of the chain, and targets and codes are stored
+//     once per block.
+constexpr int kQuadRows = 4, kQuadWaves = 8, kQuadMaxN = 4096;
+
+// The stripe's errors by row, the waves' transposes, and the count of complete quarter blocks.
+template <int NMAX>
+struct QuadLds {
+  float e[kQuadRows][NMAX + 4];  // rows 4 banks apart
+  float st[kQuadWaves][kQuadRows][64 + 4];
+  int done;
+};
+
+// a / b for b in div_box and a == 0 or in div_box, up to the sign of a zero (div_by).
+__device__ __forceinline__ float quad_div(float a, float b, float y) {
+  float q = a * y;
+  q = __fmaf_rn(__fmaf_rn(-b, q, a), y, q);
+  return __fmaf_rn(__fmaf_rn(-b, q, a), y, q);
+}
+
+// The value of lane A of each 16-lane row, in all its lanes.
+template <int A>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + A, 0xF, 0xF, true));
+}
+
+// One lane's view of the block being swept: its four columns 16 k + g of row r.
+struct QuadBlock {
+  float t[4];         // targets, then (swept) the values that were quantized
+  float dl[4], ml[4]; // committed grid step and offset
+  float y[4];         // reciprocal of the step
+  float e[4], q[4];   // errors and codes of swept columns
+  float dg, yd;       // diagonal entry of block column l and its reciprocal
+  float u[64][4];     // U[cb][16 k + g], zero where that column is not after cb (k >= cb / 16)
+};
+
+// The error of target t on the step dl (reciprocal y) and offset ml, diagonal entry d
+// (reciprocal yd): quantize_col on shared reciprocals, for operands in their range.
+__device__ __forceinline__ float quad_error(float t, float dl, float y, float ml, bool nz, float d,
+                                            float yd, float lo, float hi, float* qf) {
+  const float v = quad_div(t + ml, dl, y);
+  *qf = __builtin_rintf(__builtin_amdgcn_fmed3f(v, lo, hi));
+  const float ev = quad_div(t - (dl * *qf - ml), d, yd);
+  return nz ? ev : 0.0f;
+}
+
+// Columns 16 I + A .. 16 I + 15 on the float path: every lane forms its own column's error,
+// and the row takes the owner's. A swept column's own register keeps its value (it subtracts
+// e * 0).
+template <int I, int A>
+__device__ __forceinline__ void quad_cols(QuadBlock& b, float dl, bool nz, float lo, float hi) {
+  constexpr int cb = 16 * I + A;
+  const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(b.dg), cb));
+  const float yd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(b.yd), cb));
+  float qf;
+  const float e = quad_error(b.t[I], dl, b.y[I], b.ml[I], nz, d, yd, lo, hi, &qf);
+#pragma unroll
+  for (int k = I + (A == 15 ? 1 : 0); k < 4; ++k) b.t[k] = b.t[k] - row_bcast<A>(e) * b.u[cb][k];
+  if constexpr (A < 15) quad_cols<I, A + 1>(b, dl, nz, lo, hi);
+}
+
+// Quarter block I: columns 16 I .. 16 I + 15. fast: every step and diagonal entry of the block
+// is in the range the shared reciprocals need.
+template <int I>
+__device__ __forceinline__ void quad_quarter(const SweepTask& tk, int i1, int l, bool fast,
+                                             QuadBlock& b) {
+  const int g = l & 15;
+  if (fast) {
+    // a zero step gives code 0 and no error (ef.py:205-207): step 1 with a zero reciprocal
+    const bool nz = b.dl[I] != 0.0f;
+    const float dl = nz ? b.dl[I] : 1.0f, lo = (float)tk.lo, hi = (float)tk.hi;
+    float keep[4];
+#pragma unroll
+    for (int k = I; k < 4; ++k) keep[k] = b.t[k];
+    quad_cols<I, 0>(b, dl, nz, lo, hi);
+    // each lane's own column once more, from the value it was swept with, for its error and
+    // code and for the ranges: |t + ml| < 2^20 |dl| bounds the code's quotient (a NaN or an
+    // infinity anywhere in the row ends up in a value that fails it), and an error's numerator
+    // is zero or at least 2^-40 (at most 2^40 with the first bound and |dl| <= 2^18)
+    const float d = __shfl(b.dg, 16 * I + g), yd = __shfl(b.yd, 16 * I + g);
+    b.e[I] = quad_error(b.t[I], dl, b.y[I], b.ml[I], nz, d, yd, lo, hi, &b.q[I]);
+    const float a2 = b.t[I] - (dl * b.q[I] - b.ml[I]);
+    const bool bad = !(fabsf(b.t[I] + b.ml[I]) < 0x1p20f * fabsf(dl)) |
+                     (nz & (fabsf(a2) < 0x1p-40f) & (a2 != 0.0f));
+    if (!__any(bad)) return;
+#pragma unroll
+    for (int k = I; k < 4; ++k) b.t[k] = keep[k];
+  }
+  const GlobF ub = (GlobF)(tk.U + (int64_t)i1 * tk.n + i1);
+#pragma unroll 1
+  for (int a = 0; a < 16; ++a) {
+    const int cb = 16 * I + a;
+    const float d = __shfl(b.dg, cb);
+    float e;
+    int q;
+    quantize_col(tk, b.t[I], b.dl[I], b.ml[I], d, e, q);
+    if (g == a) {
+      b.e[I] = e;
+      b.q[I] = (float)q;
+    }
+    e = __shfl(e, (l & 48) | a);
+#pragma unroll
+    for (int k = I; k < 4; ++k) {
+      const float u = ub[(int64_t)cb * tk.n + 16 * k + g];
+      if (16 * k + g > cb) b.t[k] = b.t[k] - e * u;
+    }
+  }
+}
+
+// Wait (bounded, as wait_blocks, in sleeps of about 64 clocks) until more than c quarter
+// blocks are complete; returns their count.
+__device__ __forceinline__ int wait_quarters(int* done, int c, int limit, int* status, int lane) {
+  int v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  for (int64_t spins = 0; v <= c && spins < 4 * (int64_t)limit; ++spins) {
+    __builtin_amdgcn_s_sleep(1);
+    v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  v = __builtin_amdgcn_readfirstlane(v);
+  if (v <= c) {
+    if (lane == 0) __hip_atomic_fetch_or(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return c + 1;
+  }
+  return v;
+}
+
+// Wave w of a stripe owns blocks w, w + W, ...; every element receives its updates one at a
+// time in ascending column order, and blocks complete in order, as in ef_sweep_pipe_kernel.
+template <int NMAX>
+__global__ __launch_bounds__(64 * kQuadWaves, 2) void ef_sweep_quad_kernel(
+    const SweepTask* __restrict__ tasks, int count, int total, int xcd_runs, int wait_limit, int* status) {
+  int ti;
+  const int stripe = sweep_item(tasks, count, total, xcd_runs != 0, &ti);
+  if (stripe < 0) return;  // uniform over the workgroup
+  const SweepTask tk = tasks[ti];
+  const int row0 = stripe * kQuadRows;
+  if (row0 >= tk.nrow) return;
+  __shared__ __align__(16) QuadLds<NMAX> s;
+  if (threadIdx.x == 0) s.done = 0;
+  __syncthreads();
+  const int W = (int)blockDim.x / 64;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
+  const int l = (int)threadIdx.x & 63, r = l >> 4, g = l & 15;
+  const int nrow = tk.nrow, n = tk.n;
+  // rows past the last one repeat it and store its values again
+  const int rr = min(row0 + r, nrow - 1);
+  const int nblocks = n / 64;
+  float (*st)[64 + 4] = s.st[wv];
+  for (int bk = wv; bk < nblocks; bk += W) {
+    const int i1 = 64 * bk;
+    QuadBlock b;
+    // in the MFMA layout lane l is column l and register v row v
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4 t;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) t[v] = ld_lane(tk.WpT, (int64_t)(i1 + l) * nrow + min(row0 + v, nrow - 1));
+    b.dg = ld_lane(tk.U, (int64_t)(i1 + l) * n + i1 + l);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t o = (int64_t)tk.sbidx[i1 + 16 * k + g] * nrow + rr;
+      b.dl[k] = ld_lane(tk.dlT, o);
+      b.ml[k] = tk.mlT ? ld_lane(tk.mlT, o) : 0.0f;
+    }
+    const auto rt = __builtin_amdgcn_make_buffer_rsrc((void*)(tk.U + (int64_t)i1 * n + i1), 0, 0x7fffffff,
+                                                      0x00020000);
+    const auto load_tile = [&](int c0, int c1) {  // tile rows c0 .. c1 - 1
+#pragma unroll
+      for (int cb = 0; cb < 64; ++cb)
+        if (cb >= c0 && cb < c1) {
+#pragma unroll
+          for (int k = cb / 16; k < 4; ++k)
+            b.u[cb][k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rt, 4 * g + 64 * k, 4 * cb * n, 0));
+        }
+    };
+    const auto mask_tile = [&](int c0, int c1) {  // no entry for columns up to the row's own
+#pragma unroll
+      for (int cb = 0; cb < 64; ++cb)
+        if (cb >= c0 && cb < c1) b.u[cb][cb / 16] = g > cb % 16 ? b.u[cb][cb / 16] : 0.0f;
+    };
+    // the first half of the tile is in flight under the earlier blocks' updates, the second
+    // (48 registers that the updates' buffers hold until then) under the first half's sweep
+    load_tile(0, 32);
+    // updates of quarter blocks q0 .. q1 - 1, U loaded half a quarter (8 columns) ahead
+    int avail = 0;
+    const auto cross = [&](int q0, int q1) {
+      if (q0 >= q1) return;
+      float u[2][8];
+      const auto load = [&](int h, float (&d)[8]) {
+        const auto ru = __builtin_amdgcn_make_buffer_rsrc((void*)(tk.U + (int64_t)8 * h * n + i1), 0,
+                                                          0x7fffffff, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          d[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ru, 4 * l, 4 * j * n, 0));
+      };
+      const auto apply = [&](int h, const float (&ug)[8]) {
+        f4 e[2];  // lane l: the errors of row l % 4
+#pragma unroll
+        for (int j = 0; j < 2; ++j) e[j] = *reinterpret_cast<const f4*>(&s.e[l & 3][8 * h + 4 * j]);
+        // the products of four columns ahead of their subtractions, so none waits for its own
+#pragma unroll
+        for (int h4 = 0; h4 < 2; ++h4) {
+          f4 p[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            p[j] = __builtin_amdgcn_mfma_f32_4x4x1f32(e[h4][j], ug[4 * h4 + j], f4{0, 0, 0, 0}, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) t = t - p[j];
+        }
+      };
+      load(2 * q0, u[0]);
+      for (int q = q0; q < q1; ++q) {
+        load(2 * q + 1, u[1]);
+        if (avail <= q) avail = wait_quarters(&s.done, q, wait_limit, status, l);
+        apply(2 * q, u[0]);
+        load(q + 1 < q1 ? 2 * q + 2 : 2 * q + 1, u[0]);  // past the end: valid rows, never used
+        apply(2 * q + 1, u[1]);
+      }
+    };
+    cross(0, 4 * (bk - 1));
+    // off the chain: the tile's mask, the reciprocals and their ranges
+    bool ok = div_box(b.dg);
+    b.yd = div_recip(b.dg);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float m = fabsf(b.dl[k]);
+      ok = ok & ((m == 0.0f) | ((m >= 0x1p-25f) & (m <= 0x1p18f)));
+      b.y[k] = m == 0.0f ? 0.0f : div_recip(b.dl[k]);
+    }
+    mask_tile(0, 32);
+    const bool fast = __all(ok);
+    __builtin_amdgcn_s_setprio(3);  // the chain's wave issues before the others of its SIMD
+    cross(bk > 0 ? 4 * (bk - 1) : 0, 4 * bk);
+    load_tile(32, 64);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) st[v][l] = t[v];
+    wave_lds_fence();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b.t[k] = st[r][16 * k + g];
+    wave_lds_fence();
+    const auto publish = [&](int k) {
+      s.e[r][i1 + 16 * k + g] = b.e[k];
+      // a maximum, not a store: after a wait gave up, a late wave must not move the count back
+      if (l == 0) __hip_atomic_fetch_max(&s.done, 4 * bk + k + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    quad_quarter<0>(tk, i1, l, fast, b);
+    publish(0);
+    quad_quarter<1>(tk, i1, l, fast, b);
+    publish(1);
+    mask_tile(32, 64);
+    quad_quarter<2>(tk, i1, l, fast, b);
+    publish(2);
+    quad_quarter<3>(tk, i1, l, fast, b);
+    publish(3);
+    __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t o = (int64_t)(i1 + 16 * k + g) * nrow + rr;
+      ((GlobFw)tk.WcurT)[o] = b.t[k];
+      ((GlobBw)tk.LT)[o] = (uint8_t)((int)b.q[k] - tk.lo);
+    }
+  }
+}
+
 // MFMA mode. One wave per 64-row stripe (grid: x = stripe, y = task).
 // Cross-block updates of a block are one GEMM, acc[64 x B] = E[64 x i1] *
 // U[i1 x B], on v_mfma_f32_32x32x2f32 (A = E from the column-major error
@@ -1353,11 +1635,12 @@ int ef_encode_batch(const cp_ef_tensor* ts, int count, int n_iter, int mode, voi
   // two-per-SIMD slots and every tensor has a 64-column block per wave. 32-row stripes
   // halve the in-block quantization chain per row, so they are taken whenever some W
   // fills at least 1536 of those slots; otherwise 16-row stripes, which double the waves.
-  int64_t stripes32 = 0, stripes16 = 0;
+  int64_t stripes32 = 0, stripes16 = 0, stripes4 = 0;
   int min_blocks = 1 << 30;
   for (int i = 0; i < count; ++i) {
     stripes32 += (ts[i].nrow + 31) / 32;
     stripes16 += (ts[i].nrow + 15) / 16;
+    stripes4 += (ts[i].nrow + kQuadRows - 1) / kQuadRows;
     min_blocks = std::min(min_blocks, (int)(ts[i].n / 64));
   }
   const auto fill = [&](int64_t stripes) {
@@ -1365,10 +1648,23 @@ int ef_encode_batch(const cp_ef_tensor* ts, int count, int n_iter, int mode, voi
     while (w < 8 && stripes * 2 * w <= 2048 && 2 * w <= min_blocks) w *= 2;
     return w;
   };
+  // Quad stripes while their chain, not the arithmetic, is the call's time. Measured per sweep
+  // (quad / 16- or 32-row stripes, us): at most one stripe per CU, eight waves each: n = 1024
+  // 95 / 283, 4096 681 / 1642; two per CU, four waves: 1024 139 / 283, 4096 1199 / 1643;
+  // four per CU, two waves: 512 89 / 142, 1024 230 / 286, but 2048 1226 / 632. A wave needs a
+  // second block to be worth its slot (n = 512: four waves 48, eight 51).
+  const auto quad_waves = [&] {
+    int w = stripes4 <= 256 ? 8 : stripes4 <= 512 ? 4 : 2;
+    while (w > 1 && 2 * w > min_blocks) w /= 2;
+    return w;
+  };
   int RS, waves = 1;
   {
     const int w32 = fill(stripes32);
-    if (stripes32 * w32 >= 1536) {
+    if (mode == CP_EF_EXACT && max_n <= kQuadMaxN && stripes4 <= (max_n <= 1024 ? 1024 : 512)) {
+      RS = kQuadRows;
+      waves = quad_waves();
+    } else if (stripes32 * w32 >= 1536) {
       RS = 32;
       waves = w32;
     } else {
@@ -1377,11 +1673,14 @@ int ef_encode_batch(const cp_ef_tensor* ts, int count, int n_iter, int mode, voi
     }
   }
   if (mode == CP_EF_EXACT) {
-    if (const char* e = getenv("CP_EF_SWEEP_ROWS")) {  // tuning override: 16 or 32
+    if (const char* e = getenv("CP_EF_SWEEP_ROWS")) {  // tuning override: 4, 16 or 32
       const int r = atoi(e);
       if (r == 16 || r == 32) {
         RS = r;
         waves = fill(r == 32 ? stripes32 : stripes16);
+      } else if (r == kQuadRows && max_n <= kQuadMaxN) {
+        RS = r;
+        waves = quad_waves();
       }
     }
     if (const char* e = getenv("CP_EF_SWEEP_WAVES")) {  // tuning override: 1, 2, 4 or 8
@@ -1440,7 +1739,14 @@ int ef_encode_batch(const cp_ef_tensor* ts, int count, int n_iter, int mode, voi
     g_sweep_shape[2] = mode;
     if (mode == CP_EF_EXACT_VALU)
       ef_sweep_exact_kernel<BLK><<<dim3((unsigned)((max_rows + 255) / 256), (unsigned)count), 256, 0, st>>>(dtasks);
-    else if (mode == CP_EF_EXACT && waves == 1 && RS == 32)
+    else if (mode == CP_EF_EXACT && RS == kQuadRows) {
+      const unsigned g = (unsigned)(8 * ((total_stripes + 7) / 8));
+      const int xr = same_n ? 1 : 0, ns = (int)total_stripes;
+      if (max_n <= 1024)
+        ef_sweep_quad_kernel<1024><<<g, 64 * waves, 0, st>>>(dtasks, count, ns, xr, g_wait_limit, dstatus);
+      else
+        ef_sweep_quad_kernel<kQuadMaxN><<<g, 64 * waves, 0, st>>>(dtasks, count, ns, xr, g_wait_limit, dstatus);
+    } else if (mode == CP_EF_EXACT && waves == 1 && RS == 32)
       ef_sweep_rows_kernel<32><<<(unsigned)(8 * ((total_stripes + 7) / 8)), 64, 0, st>>>(
           dtasks, count, (int)total_stripes, same_n ? 1 : 0);
     else if (mode == CP_EF_EXACT && waves == 1)

@@ -334,6 +334,39 @@ def test_sweep_waves_per_stripe_bit_exact(ef, rows, waves, monkeypatch):
         assert (mode, rs[0], wv[0]) == (_lib.CP_EF_EXACT, int(rows), want_w)
 
 
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
+def test_quad_stripes_bit_exact(ef, waves, monkeypatch):
+    """Four-row stripes against the oracle: every wave count, rows that do not fill a stripe,
+    one block per wave and several rounds, both LDS sizes; and operands outside the range of
+    the shared reciprocals, where a quarter block is swept again by the general expressions:
+    rows of 1e-13 (errors below 2^-40), of 1e6 (steps above 2^18; there the affine fits' sums
+    leave the oracle's float32 path, so for the symmetric types), zero rows and columns (zero
+    steps) and -0.0."""
+    monkeypatch.setenv("CP_EF_SWEEP_ROWS", "4")
+    monkeypatch.setenv("CP_EF_SWEEP_WAVES", waves)
+    specs = [(41, 1024, "Q2_K", 71), (3, 256, "Q4_K", 72), (10, 1280, "Q6_K", 73),
+             (16, 512, "Q3_K", 74), (5, 768, "Q5_K", 75)]
+    for W, tt, qw, H, order, U in _oracle_items(specs):
+        _say(f"quad, waves {waves}: {tt} {W.shape}")
+        W[0] *= F32(1e-13)
+        W[1] *= F32(1e6 if tt in ("Q3_K", "Q6_K") else 1e4)
+        W[2, :300] = 0.0
+        W[2, 300:] = -0.0
+        W[-1, ::3] = 0.0
+        with np.errstate(all="ignore"):
+            want_raw, want_rec = E.ef_encode(W, tt, qw, H, n_iter=2, U=U, order=order)
+        item = {"ttype": tt, "x": torch.from_numpy(W).cuda(), "qw": torch.from_numpy(qw).cuda(),
+                "U": torch.from_numpy(U).cuda(),
+                "order": torch.from_numpy(order.astype(np.int32)).cuda()}
+        (raw, rec), = ef.ef_encode_dev([item], 2)
+        bad = np.nonzero((raw.cpu().numpy() != want_raw).any(1))[0]
+        assert bad.size == 0, f"{tt}: rows {bad} differ"
+        assert np.array_equal(rec.cpu().numpy(), want_rec, equal_nan=True)  # 1e6 overflows fp16
+        rs, wv = (ctypes.c_int * 1)(), (ctypes.c_int * 1)()
+        _lib.load().cp_ef_last_sweep(ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(wv, ctypes.c_void_p))
+        assert rs[0] == 4
+
+
 def _codes(tt, raw, nrow, n):
     return K.stored_codes(tt, raw).reshape(nrow, n)
 
