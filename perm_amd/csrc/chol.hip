@@ -51,10 +51,11 @@ constexpr int KC = 1024;
 // op(B) = B [K,N] or, with BT, B^T for B stored [N,K]. Batched over blockIdx.z
 // as z = z1 * nz2 + z2 with separate strides per level.
 //
-// Block tile 64 x 64 or 128 x 128, K tile 16, 4 waves each building a 64-column
-// slab from v_mfma_f64_16x16x4f64: stacked along M for 64 x 64 (16 x 64 each), a
-// 2 x 2 grid for 128 x 128 (64 x 64 each, half the LDS fragment reads per MFMA of
-// the stacked form). The next K tile is fetched into
+// Block tile 32 x 32, 64 x 64 or 128 x 128, K tile 16, 4 waves building it from
+// v_mfma_f64_16x16x4f64: 16-row slabs stacked along M for 64 x 64 (16 x 64 each), a
+// 2 x 2 grid for 32 x 32 (16 x 16 each) and 128 x 128 (64 x 64 each, half the LDS
+// fragment reads per MFMA of the stacked form). Every output sums its K range in the same
+// order for any tile. The next K tile is fetched into
 // registers while the current one is multiplied, then stored into the other half
 // of a double-buffered LDS, so one barrier separates K tiles. The operands of one
 // MFMA step s are read from LDS just before its MFMAs, which keeps the 128 x 128
@@ -135,12 +136,13 @@ struct GemmLds {
 template <bool BT, int BM, int BN, bool VEC>
 __device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, int bz,
                                             GemmLds<BT, BM, BN>& lds) {
-  // waves: stacked along M for BN = 64 (each BM/4 x 64), a 2 x 2 grid for BN = 128
-  // (each BM/2 x 64); fragments of one MFMA step s are read from LDS at a time
-  constexpr int WN = BN / 64;
+  // waves: stacked along M for BN = 64 (each BM/4 x 64), a 2 x 2 grid for BN = 32 and 128
+  // (each BM/2 x BN/2); fragments of one MFMA step s are read from LDS at a time
+  constexpr int WC = BN < 64 ? 16 : 64;  // columns of a wave
+  constexpr int WN = BN / WC;
   constexpr int WM = 4 / WN;
   constexpr int TI = BM / WM / 16;  // 16-row MFMA tiles per wave
-  constexpr int TJ = 4;             // 16-column MFMA tiles per wave (64 columns)
+  constexpr int TJ = WC / 16;       // 16-column MFMA tiles per wave
   constexpr int AQ = BM / 32;  // A-tile pairs fetched per thread
   constexpr int BQ = BN / 32;  // B-tile pairs fetched per thread
   auto& As = lds.As;
@@ -150,7 +152,7 @@ __device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, i
   const double* B = g.B + z1 * g.sB1 + z2 * g.sB2;
   double* C = g.C + z1 * g.sC1 + z2 * g.sC2;
   const int t = threadIdx.x, l = t & 63, w = t >> 6;
-  const int wm = (w % WM) * (BM / WM), wn = (w / WM) * 64;
+  const int wm = (w % WM) * (BM / WM), wn = (w / WM) * WC;
   const int lr = l & 15, lg = l >> 4;
   const int tr = t >> 3, tk = (t & 7) * 2;
   const int nr = t / (BN / 2), nc = (t % (BN / 2)) * 2;
@@ -299,7 +301,7 @@ static int dgemm(const GemmArgs& a0, int nz1, bool bt, hipStream_t st) {
   // CU): there the larger tile's lower L2 traffic per MFMA wins.
   // A triangular operand folds the grid: a block takes a tile and its mirror.
   const int64_t z = (int64_t)nz1 * a0.nz2;
-  const int fold = (a0.tri & 1) ? 1 : ((a0.tri & 2) ? 2 : 0);
+  int fold = (a0.tri & 1) ? 1 : ((a0.tri & 2) ? 2 : 0);
   auto blocks = [&](int tm, int tn) {
     const int64_t r = (a0.M + tm - 1) / tm, c = (a0.N + tn - 1) / tn;
     return (fold == 1 ? (r + 1) / 2 : r) * (fold == 2 ? (c + 1) / 2 : c) * z;
@@ -307,7 +309,18 @@ static int dgemm(const GemmArgs& a0, int nz1, bool bt, hipStream_t st) {
   const int kblock = a0.kc > 0 ? min(a0.kc, a0.K) : a0.K;  // K of one block's loop
   const bool wide = !g_compact_tiles && a0.M >= 128 && a0.N >= 128 && kblock >= 4096 &&
                     blocks(128, 128) >= 512;
-  const int bm = wide ? 128 : 64, bn = bm;
+  // 32 x 32 tiles (52 VGPRs, 18 KB) for products of at most 2048 64 x 64 tiles, where larger
+  // tiles leave CUs idle or hold one wave per SIMD (a K tile then costs a 64 x 64 block
+  // 0.8-1 us against 0.43 us of MFMAs). Factor alone, 64 x 64 / 32 x 32 up to 512 / 2048 /
+  // 8192 tiles, us: n = 1024 856 / 736 / 741 / 740; 2000 1865 / 1563 / 1569 / 1565; 4096
+  // 3776 / 3534 / 3582 / 3555; 28 x 3072 14294 / 14132 / 13821 / 14197; 14336 43.4 / 43.1 /
+  // 44.7 ms (2048 and 8192). Grids that stay within 512 blocks are not folded: their blocks
+  // all run at once, so a mirror only lengthens a block (1024: 755 -> 740).
+  const int64_t tiles64 = (int64_t)((a0.M + 63) / 64) * ((a0.N + 63) / 64) * z;
+  // A product written over its own A operand (the panel: N = 64) needs one block per row tile.
+  const bool small = tiles64 <= 2048 && a0.C != a0.A;
+  if (tiles64 * (small ? 4 : 1) <= 512) fold = 0;
+  const int bm = wide ? 128 : small ? 32 : 64, bn = bm;
   GemmArgs a = a0;
   a.fold = fold;
   a.ct = (a.N + bn - 1) / bn;
@@ -319,9 +332,13 @@ static int dgemm(const GemmArgs& a0, int nz1, bool bt, hipStream_t st) {
   if (total > (int64_t)1 << 30) return set_error(CP_ERR_SHAPE, "fp64 GEMM grid too large");
   const dim3 grid((unsigned)(8 * ((total + 7) / 8)));
   if (bt)
-    wide ? launch_gemm<true, 128, 128>(a, grid, vec, st) : launch_gemm<true, 64, 64>(a, grid, vec, st);
+    wide    ? launch_gemm<true, 128, 128>(a, grid, vec, st)
+    : small ? launch_gemm<true, 32, 32>(a, grid, vec, st)
+            : launch_gemm<true, 64, 64>(a, grid, vec, st);
   else
-    wide ? launch_gemm<false, 128, 128>(a, grid, vec, st) : launch_gemm<false, 64, 64>(a, grid, vec, st);
+    wide    ? launch_gemm<false, 128, 128>(a, grid, vec, st)
+    : small ? launch_gemm<false, 32, 32>(a, grid, vec, st)
+            : launch_gemm<false, 64, 64>(a, grid, vec, st);
   CP_LAUNCHED("fp64 GEMM launch");
   return CP_OK;
 }

@@ -242,11 +242,15 @@ def encode_size_classes(classes, n_iter=2, mode="exact", damp=0.01, act_order=Tr
     cur = torch.cuda.current_stream()
     streams = [_class_stream(k) for k in range(len(classes))]
     facs = []
-    # with several classes the factorizations share the GPU with other classes' EF: their
-    # GEMMs then take the 64 x 64 tiles that fit beside the sweep's workgroups (the same
-    # results; measured 77.7 -> 73.8 ms on the 28-layer Qwen3-0.6B-shaped step)
+    # with several classes the factorizations share the GPU with other classes' EF. Beside wide
+    # ones (n > 4096, the sizes that would take 128 x 128 tiles) or large batches they keep to
+    # the tiles and launches that fit beside the sweep's workgroups; few narrow matrices take
+    # the fused steps and the look-ahead stream instead. The same results either way. Kept /
+    # taken: Llama-3-8B layer 120.8 / 121.9 ms, Qwen3-0.6B layers: 1 6.87 / 6.48 ms, 4 (8
+    # matrices in the largest class) 12.9 / 12.9, 8 20.0 / 21.6, 14 33.5 / 34.0, 28 equal
     lib = _lib.load()
-    lib.cp_chol_compact_tiles(1 if len(classes) > 1 else 0)
+    wide = any(Hb.shape[-1] > 4096 or Hb.shape[0] > 8 for Hb, _ in classes)
+    lib.cp_chol_compact_tiles(1 if len(classes) > 1 and wide else 0)
     try:
         for (Hb, _), s in zip(classes, streams):
             s.wait_stream(cur)

@@ -88,6 +88,21 @@ def test_factor_matches_closed_form(ef, n):
     assert np.abs(U.T @ U @ Hd - np.eye(n)).max() < 1e-9
 
 
+@pytest.mark.parametrize("n", [31, 33, 95, 129, 287, 544])
+def test_factor_does_not_depend_on_the_tiles_in_a_batch(ef, n):
+    """Row and column counts around the 32 x 32 tiles' edges, alone (fused steps, unfolded
+    grids) and seven at a time (separate launches, the panel written over its own operand):
+    the same U bit for bit, and the closed form's."""
+    H = np.stack([correlated_hessian(n, 4 * n, seed=n + z) for z in range(7)])
+    order = np.stack([np.arange(n)] * 7)
+    Ub, _ = ef.factor_dev(torch.from_numpy(H).cuda(), order, 0.01, out_dtype=torch.float64)
+    for z in (0, 6):
+        U1, _ = ef.factor_dev(torch.from_numpy(H[z]).cuda(), order[z], 0.01, out_dtype=torch.float64)
+        assert torch.equal(U1, Ub[z])
+        want = E.inv_upper_factor(H[z], 0.01)
+        assert np.abs(U1.cpu().numpy() - want).max() / np.abs(want).max() < 1e-11  # as the closed form's
+
+
 @pytest.mark.parametrize("n,N,kind", [(3072, 65536, "student-t"), (4096, 131072, "outliers"),
                                       (14336, 131072, "outliers")])
 def test_factor_matches_library_at_config_sizes(ef, n, N, kind):
