@@ -13,8 +13,8 @@
 //  bf16: lower-triangle 256 x 256 tiles on v_mfma_f32_32x32x16_bf16, operands
 //        read transposed from LDS (hess_bf16_tri_kernel), then a pass that
 //        reduces the splits and mirrors the lower triangle into the upper one;
-//  f32:  128 x 128 tiles on v_mfma_f32_32x32x2f32, which takes one row t per
-//        lane, so the [t][i] panel is used as loaded.
+//  f32:  lower-triangle 128 x 128 tiles on v_mfma_f32_32x32x2f32, which takes one row t
+//        per lane, so the [t][i] panel is used as loaded.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -392,41 +392,90 @@ __global__ __launch_bounds__(256) void hess_tri_reduce_kernel(const HessJobs job
 }
 
 // ---------------------------------------------------------------- f32 input
-// part == nullptr (one row split): the workgroup adds its tile into H. Otherwise
-// it stores the tile into split blockIdx.z's full [d, d] partial in part, for
-// hess_f32_reduce_kernel.
-__global__ __launch_bounds__(256) void hess_f32_kernel(const float* __restrict__ X, int64_t N, int d,
-                                                       int64_t rows_per_split, float* __restrict__ H,
-                                                       float* __restrict__ part) {
-  __shared__ float sA[KT][HT + 4];
-  __shared__ float sB[KT][HT + 4];
-  const int i0 = blockIdx.y * HT, j0 = blockIdx.x * HT;
-  const int64_t r0 = (int64_t)blockIdx.z * rows_per_split;
-  const int64_t r1 = min(N, r0 + rows_per_split);
+// Lower-triangle 128 x 128 tiles on v_mfma_f32_32x32x2f32, split-K over rows of X; the
+// products of the two triangles are equal bit for bit (the factors commute), so each tile
+// serves both. Four waves of 64 x 64. Bound by the f32 matrix rate (64 cycles per 4096
+// flops): rows come 32 at a time through raw buffer loads one stage ahead (rows past the
+// split and columns past d read zeros, so any d takes the same loop) into a double-buffered
+// LDS panel pair, one barrier per stage, two workgroups per CU. Full square tiles loaded with
+// bounds branches and no stage in flight ran [8192, 1024] in 345 us (25 TFLOP/s of the
+// triangle); this takes 88 us and 9 for the splits' sum (340 -> 97 us a call, 88 TFLOP/s).
+//
+// part: split s of tile k goes to slot (s, k) for hess_f32_reduce_kernel. part == nullptr
+// (one split): the workgroup adds its tile into H, above the diagonal transposed.
+constexpr int FCH = KT * HT / 256;  // floats per thread, panel and stage
+constexpr int kFlush = 8;           // stages summed in one chain: 256 rows
+
+__global__ __launch_bounds__(256, 2) void hess_f32_kernel(const float* __restrict__ X, int64_t N, int d,
+                                                          int ntiles, int splits, int64_t rows_per_split,
+                                                          float* __restrict__ H, float* __restrict__ part) {
+  __shared__ float sP[2][2][KT][HT + 4];  // [buffer][panel]
+  const int total = ntiles * splits, per = (total + 7) / 8;
+  // an XCD's workgroups share rows of X (hess_bf16_tri_kernel)
+  const int item = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (item >= total) return;
+  const int split = item / ntiles, tile = item - split * ntiles;
+  int ti = (int)((sqrtf(8.0f * (float)tile + 1.0f) - 1.0f) * 0.5f);
+  while (ti * (ti + 1) / 2 > tile) --ti;
+  while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
+  const int tj = tile - ti * (ti + 1) / 2;
+  const int i0 = ti * HT, j0 = tj * HT;
+  const bool diag = ti == tj;
+  const int64_t r0 = (int64_t)split * rows_per_split;
+  const int nrows = (int)(min(N, r0 + rows_per_split) - r0);
+  if (nrows <= 0) return;  // the host leaves no split without rows
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int wm = (w >> 1) * 64, wn = (w & 1) * 64;
-  f32x16 acc[2][2];
+  // thread: column tid % 128 of both panels, rows tid / 128 + 2 q
+  const uint32_t rowb = 4u * (uint32_t)d;
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(X + r0 * d), 0, (int)((uint32_t)nrows * rowb), 0x00020000);
+  const int c = tid & (HT - 1), rr = tid >> 7;
+  const uint32_t oi = i0 + c < d ? (uint32_t)rr * rowb + 4u * (uint32_t)(i0 + c) : kOob;
+  const uint32_t oj = j0 + c < d ? (uint32_t)rr * rowb + 4u * (uint32_t)(j0 + c) : kOob;
+  float gi[FCH], gj[FCH];
+  // the whole offset in the lane's register: the range check is against it
+  const auto fetch = [&](int st) {
+    const uint32_t so = (uint32_t)st * KT * rowb;
+#pragma unroll
+    for (int q = 0; q < FCH; ++q)
+      gi[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(oi + so + 2u * q * rowb), 0, 0));
+    if (!diag) {
+#pragma unroll
+      for (int q = 0; q < FCH; ++q)
+        gj[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(oj + so + 2u * q * rowb), 0, 0));
+    }
+  };
+  const auto stash = [&](int b) {
+#pragma unroll
+    for (int q = 0; q < FCH; ++q) sP[b][0][rr + 2 * q][c] = gi[q];
+    if (!diag) {
+#pragma unroll
+      for (int q = 0; q < FCH; ++q) sP[b][1][rr + 2 * q][c] = gj[q];
+    }
+  };
+  // sums of kFlush stages, and their running total: rounding grows with the longer of the two
+  f32x16 acc[2][2], tot[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
-  for (int64_t t0 = r0; t0 < r1; t0 += KT) {
-    for (int idx = tid; idx < KT * HT; idx += 256) {
-      int tt = idx / HT, c = idx % HT;
-      int64_t t = t0 + tt;
-      sA[tt][c] = (t < r1 && i0 + c < d) ? X[t * d + i0 + c] : 0.0f;
-      sB[tt][c] = (t < r1 && j0 + c < d) ? X[t * d + j0 + c] : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll 4
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = tot[a][b][v] = 0.0f;
+  const int stages = (nrows + KT - 1) / KT;
+  fetch(0);
+  stash(0);
+  __syncthreads();
+  for (int st = 0; st < stages; ++st) {
+    if (st + 1 < stages) fetch(st + 1);
+    const float(*pa)[HT + 4] = sP[st & 1][0];
+    const float(*pb)[HT + 4] = diag ? pa : sP[st & 1][1];
+#pragma unroll 8
     for (int k = 0; k < KT; k += 2) {
       float a[2], b[2];
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        a[x] = sA[k + (l >> 5)][wm + x * 32 + (l & 31)];
-        b[x] = sB[k + (l >> 5)][wn + x * 32 + (l & 31)];
+        a[x] = pa[k + (l >> 5)][wm + x * 32 + (l & 31)];
+        b[x] = pb[k + (l >> 5)][wn + x * 32 + (l & 31)];
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x)
@@ -434,33 +483,74 @@ __global__ __launch_bounds__(256) void hess_f32_kernel(const float* __restrict__
         for (int y = 0; y < 2; ++y)
           acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x], b[y], acc[x][y], 0, 0, 0);
     }
+    if (st % kFlush == kFlush - 1 || st + 1 == stages) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          tot[x][y] += acc[x][y];
+          acc[x][y] = 0.0f;
+        }
+    }
+    if (st + 1 < stages) stash((st + 1) & 1);
     __syncthreads();
   }
-  float* const dst = part ? part + (int64_t)blockIdx.z * d * d : H;
+  float* const slot = part + (int64_t)(split * ntiles + tile) * (HT * HT);
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        int i = i0 + wm + x * 32 + mfma32_row(v, l);
-        int j = j0 + wn + y * 32 + (l & 31);
-        if (i < d && j < d) {
-          float* p = dst + (int64_t)i * d + j;
-          *p = part ? acc[x][y][v] : *p + acc[x][y][v];
+        const int i = wm + x * 32 + mfma32_row(v, l), j = wn + y * 32 + (l & 31);
+        if (part) {
+          slot[i * HT + j] = tot[x][y][v];
+        } else if (i0 + i < d && j0 + j < d) {
+          float* p = H + (int64_t)(i0 + i) * d + j0 + j;
+          *p = *p + tot[x][y][v];
+          if (!diag) {
+            float* m = H + (int64_t)(j0 + j) * d + i0 + i;
+            *m = *m + tot[x][y][v];
+          }
         }
       }
 }
 
-// H[e] = H[e] + (p_0[e] + p_1[e] + ... + p_{splits-1}[e]): the f32 path's row
-// splits summed in split order.
-__global__ __launch_bounds__(256) void hess_f32_reduce_kernel(float* __restrict__ H, int64_t dd,
-                                                              int splits,
-                                                              const float* __restrict__ part) {
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < dd; e += (int64_t)gridDim.x * 256) {
-    float s = part[e];
-    for (int k = 1; k < splits; ++k) s += part[k * dd + e];
-    H[e] = H[e] + s;
+// The row splits' tiles summed in split order, p_0 + p_1 + ..., and added to H at (i, j) and
+// (j, i), over 32 x 32 blocks of the lower triangle (blockIdx.x, row order; small blocks, so a
+// narrow H with many splits still fills the chip); the mirror goes through LDS so both sides
+// are coalesced.
+__global__ __launch_bounds__(256) void hess_f32_reduce_kernel(float* __restrict__ H, int d, int ntiles,
+                                                              int splits, const float* __restrict__ part) {
+  __shared__ float tl[32][33];
+  int bi = (int)((sqrtf(8.0f * (float)blockIdx.x + 1.0f) - 1.0f) * 0.5f);
+  while (bi * (bi + 1) / 2 > (int)blockIdx.x) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= (int)blockIdx.x) ++bi;
+  const int bj = (int)blockIdx.x - bi * (bi + 1) / 2;
+  const int c = threadIdx.x & 31, rt = threadIdx.x >> 5;
+  const int ti = bi / 4, tj = bj / 4;
+  const int64_t slot = (int64_t)ntiles * (HT * HT);  // floats between one split's tiles
+  const float* p = part + (int64_t)(ti * (ti + 1) / 2 + tj) * (HT * HT) + ((bi % 4) * 32 + rt) * HT + (bj % 4) * 32 + c;
+  float s[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) s[q] = p[8 * q * HT];
+#pragma unroll 4
+  for (int k = 1; k < splits; ++k)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) s[q] += p[k * slot + 8 * q * HT];
+  const int j = bj * 32 + c;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = rt + 8 * q, i = bi * 32 + r;
+    tl[r][c] = s[q];
+    if (i < d && j < d) H[(int64_t)i * d + j] += s[q];
+  }
+  if (bi == bj) return;  // a diagonal block's tile is whole
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = rt + 8 * q, i = bj * 32 + r, jj = bi * 32 + c;
+    if (i < d && jj < d) H[(int64_t)i * d + jj] += tl[c][r];
   }
 }
 
@@ -498,14 +588,22 @@ static int pick_splits(int ntiles, int64_t N, int64_t d, int64_t* rows_per_split
   return (int)((N + rps - 1) / rps);  // rounding rps up may leave fewer splits with rows
 }
 
-// Row splits of the f32 kernel: about 4 workgroups per CU, each at least 512 rows.
+static int f32_tiles(int64_t d) {
+  const int64_t T = (d + HT - 1) / HT;
+  return (int)(T * (T + 1) / 2);
+}
+
+// Row splits of the f32 kernel: two workgroups per CU, each at least 128 rows. A split spans
+// at most 2^30 bytes of X, so its buffer offsets stay below 2^31.
 static int f32_splits(int64_t N, int64_t d, int64_t* rows_per_split) {
-  const int tiles = (int)((d + HT - 1) / HT);
-  const int64_t want = (1024 + (int64_t)tiles * tiles - 1) / ((int64_t)tiles * tiles);
-  const int64_t splits = want < 1 ? 1 : want;
+  const int64_t tiles = f32_tiles(d);
+  int64_t splits = 512 / tiles;
+  if (splits < 1) splits = 1;
   int64_t rps = (N + splits - 1) / splits;
-  if (rps < 512) rps = 512;
+  if (rps < 128) rps = 128;
   rps = (rps + KT - 1) / KT * KT;
+  const int64_t most = ((int64_t)1 << 30) / (4 * d) / KT * KT;  // d <= 2^20: at least 256 rows
+  if (rps > most) rps = most;
   *rows_per_split = rps;
   return (int)((N + rps - 1) / rps);
 }
@@ -526,7 +624,7 @@ static size_t hess_ws_need(int count, int x_dtype, int64_t N, int64_t d) {
   if (x_dtype == 0) {
     int64_t rps = 0;
     const int s = f32_splits(N, d, &rps);
-    return s > 1 ? (size_t)s * d * d * sizeof(float) : 0;  // jobs run one after another
+    return s > 1 ? (size_t)s * f32_tiles(d) * (HT * HT) * sizeof(float) : 0;  // jobs run one after another
   }
   size_t need = bf16_ws(count < kHessJobs ? count : kHessJobs, N, d);
   if (count > kHessJobs && count % kHessJobs) {
@@ -581,23 +679,25 @@ static int hess_bf16_batch(const void* const* X, float* const* H, int count, int
 
 static int hess_f32(const float* X, int64_t N, int64_t d, float* H, void* ws, size_t ws_bytes,
                     hipStream_t st) {
-  const int tiles = (int)((d + HT - 1) / HT);
+  const int tiles = f32_tiles(d);
   int64_t rps = 0;
   const int splits = f32_splits(N, d, &rps);
+  if ((int64_t)tiles * splits > INT32_MAX / 8)
+    return set_error(CP_ERR_SHAPE, "X [%lld, %lld] too large for one accumulation; pass fewer rows",
+                     (long long)N, (long long)d);
   float* part = nullptr;
   if (splits > 1) {
-    const size_t need = (size_t)splits * d * d * sizeof(float);
+    const size_t need = (size_t)splits * tiles * (HT * HT) * sizeof(float);
     if (!ws || ws_bytes < need)
       return set_error(CP_ERR_WORKSPACE, "Hessian workspace: need %zu bytes, have %zu", need, ws_bytes);
     part = (float*)ws;
   }
-  dim3 grid(tiles, tiles, (unsigned)splits);
-  hess_f32_kernel<<<grid, 256, 0, st>>>(X, N, (int)d, rps, H, part);
+  const int per = (tiles * splits + 7) / 8;
+  hess_f32_kernel<<<dim3(8 * per), 256, 0, st>>>(X, N, (int)d, tiles, splits, rps, H, part);
   CP_LAUNCHED("hessian launch");
   if (part) {
-    const int64_t dd = d * d;
-    const int64_t blocks = (dd + 255) / 256 < 4096 ? (dd + 255) / 256 : 4096;
-    hess_f32_reduce_kernel<<<dim3((unsigned)blocks), 256, 0, st>>>(H, dd, splits, part);
+    const int tb = (int)((d + 31) / 32);
+    hess_f32_reduce_kernel<<<dim3(tb * (tb + 1) / 2), 256, 0, st>>>(H, (int)d, tiles, splits, part);
     CP_LAUNCHED("hessian reduce");
   }
   return CP_OK;

@@ -28,6 +28,24 @@ def test_xtx_matches_closed_form(hs, dtype, N, d):
     assert torch.allclose(H, H.T, rtol=1e-4, atol=1e-5 * float(H.abs().max()))
 
 
+@pytest.mark.parametrize("N,d", [(1, 1), (31, 63), (128, 129), (129, 127), (257, 130), (4097, 65),
+                                 (1000, 387)])
+def test_float32_tiles_add_to_any_h(hs, N, d):
+    """float32 X at the edges of the 128-column tiles, the 32-row stages and the row splits (one
+    split and several), on an H that is not symmetric: both triangles keep their own values
+    under the sum. 2^-20 bounds it: sums of at most 4097 products in chains of at most 128
+    rows' MFMA steps and 33 splits stay well below 1e-6 of their norm."""
+    print(f"float32 tiles N={N} d={d}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N * 1000 + d)
+    X = torch.randn((N, d), generator=g, device="cuda")
+    H0 = torch.randn((d, d), generator=g, device="cuda")
+    want = H0.double() + X.double().T @ X.double()
+    got = hs.xtx_accumulate(X, H0.clone())
+    assert float(torch.linalg.norm(got.double() - want) / torch.linalg.norm(want)) < 2.0 ** -20
+    # both triangles took the same sum, each onto its own start
+    assert torch.equal(hs.xtx_accumulate(X), hs.xtx_accumulate(X).T)
+
+
 def test_accumulates_in_place(hs):
     g = torch.Generator(device="cuda").manual_seed(0)
     X1 = torch.randn((3000, 512), generator=g, device="cuda").to(torch.bfloat16)
