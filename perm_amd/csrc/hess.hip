@@ -495,25 +495,38 @@ __global__ __launch_bounds__(256, 2) void hess_f32_kernel(const float* __restric
     if (st + 1 < stages) stash((st + 1) & 1);
     __syncthreads();
   }
-  float* const slot = part + (int64_t)(split * ntiles + tile) * (HT * HT);
+  // the tile by rows: into its slot, or into LDS (the panels' 66 KB) on its way into H
+  float* const slot = part ? part + (int64_t)(split * ntiles + tile) * (HT * HT) : &sP[0][0][0][0];
+  const int pitch = part ? HT : HT + 4;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int i = wm + x * 32 + mfma32_row(v, l), j = wn + y * 32 + (l & 31);
-        if (part) {
-          slot[i * HT + j] = tot[x][y][v];
-        } else if (i0 + i < d && j0 + j < d) {
-          float* p = H + (int64_t)(i0 + i) * d + j0 + j;
-          *p = *p + tot[x][y][v];
-          if (!diag) {
-            float* m = H + (int64_t)(j0 + j) * d + i0 + i;
-            *m = *m + tot[x][y][v];
-          }
-        }
+      for (int v = 0; v < 16; ++v)
+        slot[(wm + x * 32 + mfma32_row(v, l)) * pitch + wn + y * 32 + (l & 31)] = tot[x][y][v];
+  if (part) return;
+  static_assert(sizeof(sP) >= HT * (HT + 4) * sizeof(float), "a tile fits the panels");
+  const float* tl = &sP[0][0][0][0];
+  __syncthreads();
+  // H's rows a0 .. + 127, columns b0 .. + 127 take t(r, c); 32 loads in flight (clamped, not
+  // branched around)
+  const auto add = [&](int a0, int b0, const auto& t) {
+    const int cc = min(b0 + c, d - 1);
+#pragma unroll
+    for (int q0 = 0; q0 < HT / 2; q0 += 32) {
+      float h[32];
+#pragma unroll
+      for (int q = 0; q < 32; ++q) h[q] = H[(int64_t)min(a0 + rr + 2 * (q0 + q), d - 1) * d + cc];
+#pragma unroll
+      for (int q = 0; q < 32; ++q) {
+        const int r = rr + 2 * (q0 + q);
+        if (a0 + r < d && b0 + c < d) H[(int64_t)(a0 + r) * d + b0 + c] = h[q] + t(r);
       }
+    }
+  };
+  add(i0, j0, [&](int r) { return tl[r * (HT + 4) + c]; });
+  if (!diag) add(j0, i0, [&](int r) { return tl[c * (HT + 4) + r]; });
 }
 
 // The row splits' tiles summed in split order, p_0 + p_1 + ..., and added to H at (i, j) and
