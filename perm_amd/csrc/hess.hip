@@ -391,6 +391,143 @@ __global__ __launch_bounds__(256) void hess_tri_reduce_kernel(const HessJobs job
   }
 }
 
+// ---------------------------------------------------------------- bf16 input, few rows
+// One hook call (a sequence of a few thousand rows, one H) gives the 256 x 256 tiles too
+// little: [2048, 1024] is 10 tiles x 8 row splits, so 80 workgroups fill a pipeline for eight
+// stages and store 21 MB of partial tiles that a second launch sums. Here a workgroup takes
+// one 64 x 64 tile of the lower triangle over all rows: its eight waves take a row range each,
+// stage their rows through LDS of their own (no barrier; rows of 192 bytes keep the
+// transposed reads conflict-free), and their sums are added in wave order in LDS. Bound by the
+// latency of a wave's stages: [2048, 1024] 31.2 -> 15.5 us a call, host work included.
+constexpr int SW = 8;                    // waves
+constexpr int SROW = 64 * 2 + 64;        // bytes per padded panel row
+constexpr int SPANEL = KS * SROW;        // 6 KB
+constexpr int SPITCH = 64 + 1;           // floats per row of a wave's sums
+
+__global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJobs jobs, int64_t N, int d) {
+  union Lds {
+    char stage[SW][2 * SPANEL];
+    float sum[SW][64][SPITCH];
+  };
+  __shared__ __align__(16) Lds lds;
+  const uint16_t* __restrict__ X = jobs.X[blockIdx.y];
+  float* __restrict__ H = jobs.H[blockIdx.y];
+  int ti = (int)((sqrtf(8.0f * (float)blockIdx.x + 1.0f) - 1.0f) * 0.5f);
+  while (ti * (ti + 1) / 2 > (int)blockIdx.x) --ti;
+  while ((ti + 1) * (ti + 2) / 2 <= (int)blockIdx.x) ++ti;
+  const int tj = (int)blockIdx.x - ti * (ti + 1) / 2;
+  const int i0 = 64 * ti, j0 = 64 * tj;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), l = (int)threadIdx.x & 63;
+  // this wave's rows: whole stages, as even as they come
+  const int64_t stages_all = (N + KS - 1) / KS, per = (stages_all + SW - 1) / SW;
+  const int64_t r0 = min(N, wv * per * KS), r1 = min(N, (wv + 1) * per * KS);
+  const int ns = (int)((r1 - r0 + KS - 1) / KS);
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.0f;
+  if (ns > 0) {
+    const uint32_t rowb = 2u * (uint32_t)d;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(X + r0 * d), 0, (int)((r1 - r0) * rowb), 0x00020000);
+    // chunk q < 4 of panel p: row l / 8 + 8 q, columns 8 (l % 8) .. + 7 (d % 8 == 0: all in or all out)
+    const uint32_t row = (uint32_t)(l >> 3) * rowb;
+    const int ci = i0 + 8 * (l & 7), cj = j0 + 8 * (l & 7);
+    const uint32_t oi = ci < d ? row + 2u * (uint32_t)ci : kOob, oj = cj < d ? row + 2u * (uint32_t)cj : kOob;
+    const auto fetch = [&](int s, uint4 (&g)[8]) {
+      const uint32_t so = (uint32_t)s * KS * rowb;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+            rs, (int)((q < 4 ? oi : oj) + so + (uint32_t)(8 * (q & 3)) * rowb), 0, 0);
+        g[q] = make_uint4(v[0], v[1], v[2], v[3]);
+      }
+    };
+    char* const base = lds.stage[wv];
+    char* const wr = base + (l >> 3) * SROW + 16 * (l & 7);
+    const int g4 = l >> 4, c4 = l & 15;
+    const char* const rd = base + (8 * (g4 >> 1) + (c4 >> 2)) * SROW + 2 * (16 * (g4 & 1) + 4 * (c4 & 3));
+    // lane l: column 32 x + l % 32 of the panel, rows 16 half + 8 (l / 32) + 0 .. 7
+    const auto operand = [&](int panel, int half, int x) {
+      const char* p = rd + panel * SPANEL + 16 * half * SROW + 64 * x;
+      const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4p)p);
+      const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4p)(p + 4 * SROW));
+      return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    // one stage: into this wave's LDS, the stage after next into the registers, and its products
+    // (the LDS serves a wave's accesses in order, so stage s + 1 overwrites what s has read)
+    const auto stage = [&](int s, uint4 (&g)[8]) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        *reinterpret_cast<uint4*>(wr + (q >> 2) * SPANEL + 8 * (q & 3) * SROW) = g[q];
+      if (s + 2 < ns) fetch(s + 2, g);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        bf16x8 a[2], b[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          a[x] = operand(0, half, x);
+          b[x] = operand(1, half, x);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y)
+            acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x], b[y], acc[x][y], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    uint4 g0[8], g1[8];
+    fetch(0, g0);
+    if (ns > 1) fetch(1, g1);
+    for (int s = 0; s < ns; s += 2) {
+      stage(s, g0);
+      if (s + 1 < ns) stage(s + 1, g1);
+    }
+  }
+  __syncthreads();  // every wave is done with its staging area
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) lds.sum[wv][32 * x + mfma32_row(v, l)][32 * y + (l & 31)] = acc[x][y][v];
+  __syncthreads();
+  // entry (r, c) of the tile: H plus the waves' sums in order, at (i, j) and, as H leaves
+  // symmetric, at (j, i); a diagonal tile's entries above the diagonal are its mirror's
+  float v[8];
+  const int c = l;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = wv + SW * q;
+    v[q] = lds.sum[0][r][c];
+#pragma unroll
+    for (int k = 1; k < SW; ++k) v[q] += lds.sum[k][r][c];
+    const int i = i0 + r, j = j0 + c;
+    if (i < d && j <= i) v[q] += H[(int64_t)i * d + j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = wv + SW * q, i = i0 + r, j = j0 + c;
+    lds.sum[0][r][c] = v[q];
+    if (i < d && j <= i) H[(int64_t)i * d + j] = v[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = wv + SW * q, i = j0 + r, j = i0 + c;  // (i, j) above the diagonal
+    if (j < d && i < j) H[(int64_t)i * d + j] = lds.sum[0][c][r];
+  }
+}
+
 // ---------------------------------------------------------------- f32 input
 // Lower-triangle 128 x 128 tiles on v_mfma_f32_32x32x2f32, split-K over rows of X; the
 // products of the two triangles are equal bit for bit (the factors commute), so each tile
@@ -623,8 +760,19 @@ static int f32_splits(int64_t N, int64_t d, int64_t* rows_per_split) {
 
 constexpr size_t kTileBytes = (size_t)BT * BT * sizeof(float);
 
+// The few-rows kernel for launches whose 64 x 64 tiles run in one round (one workgroup per CU)
+// and whose activations are small. Measured against the 256 x 256 tiles, us: [2048, 1024] 15.5 /
+// 31.2, [8192, 1024] 36 / 49, [12288, 1024] 51 / 55, [16384, 1024] 65 / 61, [32768, 384] 97 / 110,
+// [65536, 512] 209 / 123, [100, 1384] 13 / 60, [8192, 1384] 49 / 48; past one round: 4 x
+// [2048, 1024] 43 / 37, [2048, 3072] 76 / 52.
+static bool few_rows(int cn, int64_t N, int64_t d) {
+  const int64_t t64 = (d + 63) / 64;
+  return t64 * (t64 + 1) / 2 * cn <= 256 && N * d <= (int64_t)3 << 22;
+}
+
 // Workspace of one bf16 launch of cn jobs (0 when it runs as one split).
 static size_t bf16_ws(int cn, int64_t N, int64_t d) {
+  if (few_rows(cn, N, d)) return 0;
   const int T = (int)((d + BT - 1) / BT);
   const int ntiles = T * (T + 1) / 2;
   int64_t rps = 0;
@@ -665,6 +813,12 @@ static int hess_bf16_batch(const void* const* X, float* const* H, int count, int
         return set_error(CP_ERR_ALIGN, "job %d: X needs 16-byte alignment", c0 + i);
       jobs.X[i] = (const uint16_t*)X[c0 + i];
       jobs.H[i] = H[c0 + i];
+    }
+    if (few_rows(cn, N, d)) {
+      const int t64 = (int)((d + 63) / 64);
+      hess_bf16_small_kernel<<<dim3(t64 * (t64 + 1) / 2, cn), 64 * SW, 0, st>>>(jobs, N, (int)d);
+      CP_LAUNCHED("hessian launch");
+      continue;
     }
     int64_t rps = 0;
     const int splits = pick_splits(ntiles * cn, N, d, &rps);

@@ -28,6 +28,27 @@ def test_xtx_matches_closed_form(hs, dtype, N, d):
     assert torch.allclose(H, H.T, rtol=1e-4, atol=1e-5 * float(H.abs().max()))
 
 
+@pytest.mark.parametrize("N,d,jobs", [(1, 8, 1), (31, 64, 2), (33, 72, 3), (255, 136, 1), (257, 200, 1),
+                                      (2049, 1400, 1), (12288, 1024, 1), (12289, 1024, 1),
+                                      (300, 1024, 2)])
+def test_few_rows_bf16(hs, N, d, jobs):
+    """bf16 batches of few rows at the edges of the 64-column tiles, the 32-row stages and the
+    eight waves' row ranges (some without rows), on both sides of the rule that picks the
+    kernel: H's lower triangle plus the products, mirrored, whatever its upper triangle held.
+    2^-20 as for float32: chains of at most 1536 rows, then eight sums."""
+    print(f"few rows N={N} d={d} jobs={jobs}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N * 1000 + d)
+    Xs = [torch.randn((N, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(jobs)]
+    H0 = torch.tril(torch.randn((d, d), generator=g, device="cuda"))
+    upper = torch.ones_like(H0).triu(1) > 0
+    Hs = [torch.where(upper, torch.full_like(H0, float("nan")), H0) for _ in range(jobs)]
+    hs.xtx_accumulate_many(Xs, Hs)
+    for X, H in zip(Xs, Hs):
+        want = (H0 + torch.tril(H0, -1).T).double() + X.double().T @ X.double()
+        assert torch.equal(H, H.T)
+        assert float(torch.linalg.norm(H.double() - want) / torch.linalg.norm(want)) < 2.0 ** -20
+
+
 @pytest.mark.parametrize("N,d", [(1, 1), (31, 63), (128, 129), (129, 127), (257, 130), (4097, 65),
                                  (1000, 387)])
 def test_float32_tiles_add_to_any_h(hs, N, d):
