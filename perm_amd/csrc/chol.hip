@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "cp_host.h"
+#include "np_sum.h"
 
 namespace cp {
 
@@ -132,30 +133,144 @@ struct GemmLds {
   double Bs[2][BROWS][BLD];
 };
 
-// One block's tile (bx, by) of matrix bz (and its mirror when the grid folds).
+// Waves of a block: stacked along M for BN = 64 (each BM/4 x 64), a 2 x 2 grid for BN = 32 and
+// 128 (each BM/2 x BN/2).
+template <int BM, int BN>
+struct GemmWave {
+  static constexpr int WC = BN < 64 ? 16 : 64;  // columns of a wave
+  static constexpr int WN = BN / WC, WM = 4 / WN;
+  static constexpr int TI = BM / WM / 16;  // 16-row MFMA tiles per wave
+  static constexpr int TJ = WC / 16;       // 16-column MFMA tiles per wave
+  int wm, wn, lr, lg;
+  __device__ __forceinline__ GemmWave() {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    wm = (w % WM) * (BM / WM);
+    wn = (w / WM) * WC;
+    lr = l & 15;
+    lg = l >> 4;
+  }
+};
+
+template <int BM, int BN>
+using GemmAcc = dbl4[GemmWave<BM, BN>::TI][GemmWave<BM, BN>::TJ];
+
+// acc += A[bm.., kbeg..kend) op(B)[kbeg..kend, bn..], K tiles in ascending order (kbeg a multiple
+// of GBK; columns at or past klim load as zero). A caller may split a K range over calls: the
+// accumulators see the same MFMAs in the same order.
 template <bool BT, int BM, int BN, bool VEC>
-__device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, int bz,
-                                            GemmLds<BT, BM, BN>& lds) {
-  // waves: stacked along M for BN = 64 (each BM/4 x 64), a 2 x 2 grid for BN = 32 and 128
-  // (each BM/2 x BN/2); fragments of one MFMA step s are read from LDS at a time
-  constexpr int WC = BN < 64 ? 16 : 64;  // columns of a wave
-  constexpr int WN = BN / WC;
-  constexpr int WM = 4 / WN;
-  constexpr int TI = BM / WM / 16;  // 16-row MFMA tiles per wave
-  constexpr int TJ = WC / 16;       // 16-column MFMA tiles per wave
+__device__ __forceinline__ void gemm_acc(const GemmArgs& g, const double* A, const double* B, int bm, int bn,
+                                         int kbeg, int kend, int klim, GemmAcc<BM, BN>& acc,
+                                         GemmLds<BT, BM, BN>& lds) {
+  using W = GemmWave<BM, BN>;
+  constexpr int TI = W::TI, TJ = W::TJ;
   constexpr int AQ = BM / 32;  // A-tile pairs fetched per thread
   constexpr int BQ = BN / 32;  // B-tile pairs fetched per thread
   auto& As = lds.As;
   auto& Bs = lds.Bs;
+  const W wv;
+  const int wm = wv.wm, wn = wv.wn, lr = wv.lr, lg = wv.lg;
+  const int t = threadIdx.x;
+  const int tr = t >> 3, tk = (t & 7) * 2;
+  const int nr = t / (BN / 2), nc = (t % (BN / 2)) * 2;
+  const int nt = kend > kbeg ? (kend - kbeg + GBK - 1) / GBK : 0;
+
+  double2 ra[AQ], rb[BQ];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < AQ; ++q) {
+      const int r = bm + tr + 32 * q;
+      ra[q] = ld_pair<VEC>(A + (int64_t)r * g.lda + k0 + tk, r < g.M, k0 + tk, klim);
+    }
+#pragma unroll
+    for (int q = 0; q < BQ; ++q) {
+      if (BT) {
+        const int r = bn + tr + 32 * q;
+        rb[q] = ld_pair<VEC>(B + (int64_t)r * g.ldb + k0 + tk, r < g.N, k0 + tk, klim);
+      } else {
+        const int k = k0 + nr + (512 / BN) * q;
+        rb[q] = ld_pair<VEC>(B + (int64_t)k * g.ldb + bn + nc, k < klim, bn + nc, g.N);
+      }
+    }
+  };
+  auto stash = [&](int b) {
+#pragma unroll
+    for (int q = 0; q < AQ; ++q) *reinterpret_cast<double2*>(&As[b][tr + 32 * q][tk]) = ra[q];
+#pragma unroll
+    for (int q = 0; q < BQ; ++q) {
+      if (BT)
+        *reinterpret_cast<double2*>(&Bs[b][tr + 32 * q][tk]) = rb[q];
+      else
+        *reinterpret_cast<double2*>(&Bs[b][nr + (512 / BN) * q][nc]) = rb[q];
+    }
+  };
+
+  // the previous tile's last K step ended with a barrier, so its LDS reads are done
+  if (nt > 0) {
+    fetch(kbeg);
+    stash(0);
+  }
+  __syncthreads();
+  for (int it = 0; it < nt; ++it) {
+    const int b = it & 1;
+    if (it + 1 < nt) fetch(kbeg + (it + 1) * GBK);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      double af[TI], bf[TJ];
+#pragma unroll
+      for (int ti = 0; ti < TI; ++ti) af[ti] = As[b][wm + 16 * ti + lr][4 * lg + s];
+#pragma unroll
+      for (int tj = 0; tj < TJ; ++tj)
+        bf[tj] = BT ? Bs[b][wn + 16 * tj + lr][4 * lg + s] : Bs[b][4 * lg + s][wn + 16 * tj + lr];
+#pragma unroll
+      for (int ti = 0; ti < TI; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < TJ; ++tj)
+          acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[ti], bf[tj], acc[ti][tj], 0, 0, 0);
+    }
+    if (it + 1 < nt) stash(b ^ 1);
+    __syncthreads();
+  }
+}
+
+template <int BM, int BN>
+__device__ __forceinline__ void gemm_zero(GemmAcc<BM, BN>& acc) {
+#pragma unroll
+  for (int i = 0; i < GemmWave<BM, BN>::TI; ++i)
+#pragma unroll
+    for (int j = 0; j < GemmWave<BM, BN>::TJ; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
+}
+
+// C[bm.., bn..] = alpha * acc + beta * C
+template <int BM, int BN>
+__device__ __forceinline__ void gemm_store(const GemmArgs& g, double* C, int bm, int bn,
+                                           const GemmAcc<BM, BN>& acc) {
+  using W = GemmWave<BM, BN>;
+  const W wv;
+#pragma unroll
+  for (int ti = 0; ti < W::TI; ++ti)
+#pragma unroll
+    for (int tj = 0; tj < W::TJ; ++tj)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // v_mfma_f64_16x16x4f64 result: register r of lane l holds row 4r + l/16, column l%16
+        const int i = bm + wv.wm + 16 * ti + 4 * r + wv.lg;
+        const int j = bn + wv.wn + 16 * tj + wv.lr;
+        if (i < g.M && j < g.N) {
+          double* q = C + (int64_t)i * g.ldc + j;
+          const double v = g.alpha * acc[ti][tj][r];
+          *q = g.beta == 0.0 ? v : v + g.beta * *q;
+        }
+      }
+}
+
+// One block's tile (bx, by) of matrix bz (and its mirror when the grid folds).
+template <bool BT, int BM, int BN, bool VEC>
+__device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, int bz,
+                                            GemmLds<BT, BM, BN>& lds) {
   const int z1 = bz / g.nz2, z2 = bz % g.nz2;
   const double* A = g.A + z1 * g.sA1 + z2 * g.sA2;
   const double* B = g.B + z1 * g.sB1 + z2 * g.sB2;
   double* C = g.C + z1 * g.sC1 + z2 * g.sC2;
-  const int t = threadIdx.x, l = t & 63, w = t >> 6;
-  const int wm = (w % WM) * (BM / WM), wn = (w / WM) * WC;
-  const int lr = l & 15, lg = l >> 4;
-  const int tr = t >> 3, tk = (t & 7) * 2;
-  const int nr = t / (BN / 2), nc = (t % (BN / 2)) * 2;
   // A triangular operand makes a tile's K range grow with its row (tri & 1) or shrink
   // with its column (tri & 2). The block then takes a tile and its mirror, whose ranges
   // add up to the same length for every block, so no long tile is left running alone
@@ -167,13 +282,6 @@ __device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, i
     const int bm = (p && g.fold == 1 ? mir : by) * BM;
     const int bn = (p && g.fold == 2 ? mir : bx) * BN;
     if ((g.tri & 4) && bn >= bm + BM) continue;
-
-    dbl4 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-
     int kbeg = (g.tri & 2) ? (bn & ~(GBK - 1)) : 0;
     int kend = (g.tri & 1) ? min(g.K, bm + BM) : g.K;
     if (g.kc > 0) {
@@ -182,79 +290,10 @@ __device__ __forceinline__ void dgemm_block(const GemmArgs& g, int bx, int by, i
     }
     // columns at or past klim load as zero: K's end, or the end of this block's chunk
     const int klim = g.kc > 0 ? kend : g.K;
-    const int nt = kend > kbeg ? (kend - kbeg + GBK - 1) / GBK : 0;
-
-    double2 ra[AQ], rb[BQ];
-    auto fetch = [&](int k0) {
-#pragma unroll
-      for (int q = 0; q < AQ; ++q) {
-        const int r = bm + tr + 32 * q;
-        ra[q] = ld_pair<VEC>(A + (int64_t)r * g.lda + k0 + tk, r < g.M, k0 + tk, klim);
-      }
-#pragma unroll
-      for (int q = 0; q < BQ; ++q) {
-        if (BT) {
-          const int r = bn + tr + 32 * q;
-          rb[q] = ld_pair<VEC>(B + (int64_t)r * g.ldb + k0 + tk, r < g.N, k0 + tk, klim);
-        } else {
-          const int k = k0 + nr + (512 / BN) * q;
-          rb[q] = ld_pair<VEC>(B + (int64_t)k * g.ldb + bn + nc, k < klim, bn + nc, g.N);
-        }
-      }
-    };
-    auto stash = [&](int b) {
-#pragma unroll
-      for (int q = 0; q < AQ; ++q) *reinterpret_cast<double2*>(&As[b][tr + 32 * q][tk]) = ra[q];
-#pragma unroll
-      for (int q = 0; q < BQ; ++q) {
-        if (BT)
-          *reinterpret_cast<double2*>(&Bs[b][tr + 32 * q][tk]) = rb[q];
-        else
-          *reinterpret_cast<double2*>(&Bs[b][nr + (512 / BN) * q][nc]) = rb[q];
-      }
-    };
-
-    // the previous tile's last K step ended with a barrier, so its LDS reads are done
-    if (nt > 0) {
-      fetch(kbeg);
-      stash(0);
-    }
-    __syncthreads();
-    for (int it = 0; it < nt; ++it) {
-      const int b = it & 1;
-      if (it + 1 < nt) fetch(kbeg + (it + 1) * GBK);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        double af[TI], bf[TJ];
-#pragma unroll
-        for (int ti = 0; ti < TI; ++ti) af[ti] = As[b][wm + 16 * ti + lr][4 * lg + s];
-#pragma unroll
-        for (int tj = 0; tj < TJ; ++tj)
-          bf[tj] = BT ? Bs[b][wn + 16 * tj + lr][4 * lg + s] : Bs[b][4 * lg + s][wn + 16 * tj + lr];
-#pragma unroll
-        for (int ti = 0; ti < TI; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < TJ; ++tj)
-            acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[ti], bf[tj], acc[ti][tj], 0, 0, 0);
-      }
-      if (it + 1 < nt) stash(b ^ 1);
-      __syncthreads();
-    }
-#pragma unroll
-    for (int ti = 0; ti < TI; ++ti)
-#pragma unroll
-      for (int tj = 0; tj < TJ; ++tj)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          // v_mfma_f64_16x16x4f64 result: register r of lane l holds row 4r + l/16, column l%16
-          const int i = bm + wm + 16 * ti + 4 * r + lg;
-          const int j = bn + wn + 16 * tj + lr;
-          if (i < g.M && j < g.N) {
-            double* q = C + (int64_t)i * g.ldc + j;
-            const double v = g.alpha * acc[ti][tj][r];
-            *q = g.beta == 0.0 ? v : v + g.beta * *q;
-          }
-        }
+    GemmAcc<BM, BN> acc;
+    gemm_zero<BM, BN>(acc);
+    gemm_acc<BT, BM, BN, VEC>(g, A, B, bm, bn, kbeg, kend, klim, acc, lds);
+    gemm_store<BM, BN>(g, C, bm, bn, acc);
   }
 }
 
@@ -348,148 +387,50 @@ static int dgemm(const GemmArgs& a0, int nz1, bool bt, hipStream_t st) {
 // flagged by fact_shift_kernel and must never address memory outside H.
 __device__ inline int clamp_index(int p, int n) { return p < 0 ? 0 : (p >= n ? n - 1 : p); }
 
-// numpy's pairwise float64 sum of a strided vector (same recursion as the
-// float32 one: 8 accumulators up to 128 elements, halving split above).
-__device__ double pw_sum_f64(const double* a, int n, int stride) {
-  if (n < 8) {
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s = s + a[(int64_t)i * stride];
-    return s;
-  }
-  if (n <= 128) {
-    double r[8];
-    for (int j = 0; j < 8; ++j) r[j] = a[(int64_t)j * stride];
-    int i = 8;
-    for (; i < n - (n % 8); i += 8)
-      for (int j = 0; j < 8; ++j) r[j] = r[j] + a[(int64_t)(i + j) * stride];
-    double s = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
-    for (; i < n; ++i) s = s + a[(int64_t)i * stride];
-    return s;
-  }
-  int n2 = n / 2;
-  n2 -= n2 % 8;
-  return pw_sum_f64(a, n2, stride) + pw_sum_f64(a + (int64_t)n2 * stride, n - n2, stride);
-}
-
-// numpy reduces a float64 vector in chunks of 8192 values (its ufunc buffer
-// size): the pairwise recursion runs inside each chunk, and the chunk sums are
-// added left to right onto +0.0. This holds for contiguous and strided inputs
-// alike (np.diag(H) is a strided view).
-constexpr int kNpChunk = 8192;
-
-// Leaves of numpy's pairwise sum over n values, chunk by chunk and in order:
-// inside a chunk the recursion above splits until a piece has at most 128
-// values. Returns the leaf count (at most max_leaves written).
-__device__ int pw_leaves(int n, int max_leaves, int* off, int* len) {
-  int k = 0;
-  for (int c0 = 0; c0 < n; c0 += kNpChunk) {
-    int stack_off[32], stack_len[32], sp = 0;
-    stack_off[sp] = c0;
-    stack_len[sp++] = min(kNpChunk, n - c0);
-    while (sp > 0) {
-      --sp;
-      const int o = stack_off[sp], m = stack_len[sp];
-      if (m <= 128) {
-        if (k < max_leaves) {
-          off[k] = o;
-          len[k] = m;
-        }
-        ++k;
-        continue;
-      }
-      int m2 = m / 2;
-      m2 -= m2 % 8;
-      stack_off[sp] = o + m2;  // right piece below the left one: leaves come out in order
-      stack_len[sp++] = m - m2;
-      stack_off[sp] = o;
-      stack_len[sp++] = m2;
-    }
-  }
-  return k;
-}
-
-// One chunk's pairwise tree combined from its leaf sums, in the recursion's order.
-__device__ double pw_combine(int n, const double* leaf, int& k) {
-  if (n <= 128) return leaf[k++];
-  int n2 = n / 2;
-  n2 -= n2 % 8;
-  const double a = pw_combine(n2, leaf, k);
-  return a + pw_combine(n - n2, leaf, k);
-}
-
-// np.add.reduce of n float64 values from their leaf sums: chunk trees added in order.
-__device__ double np_sum_from_leaves(int n, const double* leaf) {
-  double total = 0.0;
-  int k = 0;
-  for (int c0 = 0; c0 < n; c0 += kNpChunk) total = total + pw_combine(min(kNpChunk, n - c0), leaf, k);
-  return total;
-}
-
-// np.add.reduce of n float64 values, serially.
-__device__ double np_sum_f64(const double* a, int n) {
-  double total = 0.0;
-  for (int c0 = 0; c0 < n; c0 += kNpChunk) total = total + pw_sum_f64(a + c0, min(kNpChunk, n - c0), 1);
-  return total;
-}
-
-constexpr int kShiftLeaves = 1024;  // pairwise leaves summed in parallel (n <= 131072)
+constexpr int kMarkBits = 1 << 17;  // order entries whose marks fit 16 KB of LDS
 
 // Diagonal of the act-ordered H in visiting order, then the damping shift
 // damp * mean + 1e-8 (mean replaced by 1 when not positive), as ef.py:64-69
-// computes it from np.mean(np.diag(Hp)). One block per matrix: the leaves of
-// the chunked pairwise sum run on separate threads, then one thread combines
-// them in numpy's order (same additions, same order as the serial sum).
+// computes it from np.mean(np.diag(Hp)). One block per matrix, latency-bound: the order's
+// marks are bits in LDS, and the sum runs as np_sum_block.
 //
 // The order is checked here as well: an entry outside [0, n) or a repeated one sets
-// bit 2 of fail[z] (marks: n ints of scratch per matrix, cleared here). Every
-// kernel of the factorization clamps the order's entries, so a bad order never
-// reads outside H.
+// bit 2 of fail[z] (past kMarkBits entries with marks: n ints of scratch per matrix,
+// cleared here). Every kernel of the factorization clamps the order's entries, so a bad
+// order never reads outside H.
 template <typename T>
-__global__ __launch_bounds__(256) void fact_shift_kernel(const T* H, int n, int64_t sH,
-                                                         const int* order, int64_t sO,
-                                                         const double* damp, double* diag_tmp,
-                                                         double* shift, const int* active,
-                                                         int* marks, int64_t sM, int* fail) {
-  __shared__ int loff[kShiftLeaves], llen[kShiftLeaves];
-  __shared__ double lsum[kShiftLeaves];
-  __shared__ int nleaves, bad_order;
+__global__ __launch_bounds__(1024) void fact_shift_kernel(const T* H, int n, int64_t sH,
+                                                          const int* order, int64_t sO,
+                                                          const double* damp, double* diag_tmp,
+                                                          double* shift, const int* active,
+                                                          int* marks, int64_t sM, int* fail) {
+  __shared__ NpSumLds lds;
+  __shared__ unsigned bits[kMarkBits / 32];
   const int z = blockIdx.x;
   if (active && !active[z]) return;
   const T* h = H + z * sH;
   const int* o = order ? order + z * sO : nullptr;
   double* dg = diag_tmp + (int64_t)z * n;
-  if (threadIdx.x == 0) bad_order = 0;
+  int* mk = marks + z * sM;
+  const bool in_lds = n <= kMarkBits;
   if (o) {
-    int* mk = marks + z * sM;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) mk[i] = 0;
-    __syncthreads();
-    int bad = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int p = o[i];
-      if ((unsigned)p >= (unsigned)n) bad = 1;
-      else if (atomicExch(&mk[p], 1)) bad = 1;
-    }
-    if (bad) atomicOr(&bad_order, 1);
-  }
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const int p = o ? clamp_index(o[i], n) : i;
-    dg[i] = (double)h[(int64_t)p * n + p];
-  }
-  if (threadIdx.x == 0) nleaves = pw_leaves(n, kShiftLeaves, loff, llen);
-  __syncthreads();
-  if (threadIdx.x == 0 && bad_order) fail[z] |= 2;
-  const int nl = nleaves;
-  if (nl <= kShiftLeaves) {
-    for (int k = threadIdx.x; k < nl; k += blockDim.x) lsum[k] = pw_sum_f64(dg + loff[k], llen[k], 1);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    double total;
-    if (nl <= kShiftLeaves)
-      total = np_sum_from_leaves(n, lsum);
+    if (in_lds)
+      for (int i = threadIdx.x; i < (n + 31) / 32; i += blockDim.x) bits[i] = 0;
     else
-      total = np_sum_f64(dg, n);
-    const double mean = total / (double)n;
+      for (int i = threadIdx.x; i < n; i += blockDim.x) mk[i] = 0;
+  }
+  __syncthreads();
+  int bad = 0;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const int q = o ? o[i] : i, p = clamp_index(q, n);
+    dg[i] = (double)h[(int64_t)p * n + p];
+    if (o)
+      bad |= p != q || (in_lds ? atomicOr(&bits[p >> 5], 1u << (p & 31)) >> (p & 31) & 1u
+                               : (unsigned)atomicExch(&mk[p], 1));
+  }
+  if (__syncthreads_or(bad) && threadIdx.x == 0) fail[z] |= 2;
+  const double mean = np_sum_block([=](int64_t i) { return dg[i]; }, n, lds) / (double)n;
+  if (threadIdx.x == 0) {
     const double base = mean > 0.0 ? mean : 1.0;
     shift[z] = damp[z] * base + 1e-8;
   }
@@ -805,13 +746,16 @@ __global__ __launch_bounds__(256) void fact_diag_kernel(double* A, int64_t sA, d
 // the column, the diagonal block, and the panel below it. Work items are handed out by
 // a ticket counter, matrix by matrix with the diagonal item first, so an item's diagonal
 // block always belongs to a workgroup that has already started. The diagonal item
-// updates its tile, factors and inverts it, and publishes the step in done[z] (each
+// factors and inverts its tile, and publishes the step in done[z] (each
 // thread's stores released at agent scope first); a panel item updates its tile, waits
 // for that flag (bounded: past wait_limit sleeps it sets bit 2 of fail[z] and goes on,
 // so every workgroup ends, and the host reports a timeout), then multiplies by the
-// inverse. The tile updates and products are the same block code, with the same
-// arguments, as the separate inner-update, diagonal and panel launches, so U does not
-// depend on which form ran.
+// inverse. The first panel item also updates the next step's diagonal tile, whose rows are
+// its own: the products over earlier columns run while it waits, and only those over the
+// column it has just finished are left for after, where the diagonal item's own update
+// would come before its factorization (steps 34.0 -> 31.3 us on average). The tile updates and products are the same block
+// code, over the same K tiles in the same order, as the separate inner-update, diagonal and
+// panel launches, so U does not depend on which form ran.
 struct FactStep {
   double *A, *X;
   int64_t sA;
@@ -833,19 +777,31 @@ __global__ __launch_bounds__(256, 2) void fact_step_kernel(FactStep f) {
   const int item = s_item, z = item / f.items, t = item % f.items;
   if (f.active && !f.active[z]) return;
   const int n = f.n, k = f.k, wk = n - k < NB ? n - k : NB;
-  // A[k:, k:k+wk] -= L[k:, k0:k] L[k:k+wk, k0:k]^T, tile t of 64 rows
+  // A[k:, k:k+wk] -= L[k:, k0:k] L[k:k+wk, k0:k]^T, tile t of 64 rows (tile 0: the previous
+  // step's first panel item has done it)
   const GemmArgs inner{f.A + (int64_t)k * n + f.k0, f.A + (int64_t)k * n + f.k0, f.A + (int64_t)k * n + k,
                        n - k, wk, k - f.k0, n, n, n, -1.0, 1.0, f.sA, f.sA, f.sA, 0, 0, 0, 1, 0};
-  if (k > f.k0) {
-    dgemm_block<true, 64, 64, VEC>(inner, 0, t, z, lds.g);
-    __syncthreads();  // the tile's stores before this workgroup reads it back
-  }
   if (t == 0) {
     diag_block(f.A, f.sA, f.X, f.sA, n, k, f.fail, z, lds.d);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(&f.done[z], f.step + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     return;
+  }
+  if (k > f.k0) {
+    dgemm_block<true, 64, 64, VEC>(inner, 0, t, z, lds.g);
+    __syncthreads();  // the tile's stores before this workgroup reads it back
+  }
+  // the next step's inner update of its diagonal tile, K = columns k0 .. k + 63, from row k + 64
+  const int kn = k + NB, K = kn - f.k0;
+  const bool ahead = t == 1 && K < NW;  // the next step is in this block column
+  const double* Ln = f.A + z * f.sA + (int64_t)kn * n + f.k0;
+  const GemmArgs next{Ln, Ln, nullptr, n - kn, n - kn < NB ? n - kn : NB, K, n, n, n, -1.0, 1.0,
+                      0, 0, 0, 0, 0, 0, 1, 0};
+  GemmAcc<64, 64> acc;
+  if (ahead) {
+    gemm_zero<64, 64>(acc);
+    gemm_acc<true, 64, 64, VEC>(next, Ln, Ln, 0, 0, 0, k - f.k0, K, acc, lds.g);
   }
   if (threadIdx.x == 0) {
     int v = __hip_atomic_load(&f.done[z], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -862,6 +818,11 @@ __global__ __launch_bounds__(256, 2) void fact_step_kernel(FactStep f) {
   const GemmArgs panel{f.A + (int64_t)(k + NB) * n + k, f.X + (int64_t)k * n + k, f.A + (int64_t)(k + NB) * n + k,
                        m, NB, NB, n, n, n, 1.0, 0.0, f.sA, f.sA, f.sA, 0, 0, 0, 1, 0};
   dgemm_block<true, 64, 64, VEC>(panel, 0, t - 1, z, lds.g);
+  if (ahead) {
+    __syncthreads();  // the panel tile's stores before they are read back
+    gemm_acc<true, 64, 64, VEC>(next, Ln, Ln, 0, 0, k - f.k0, K, K, acc, lds.g);
+    gemm_store<64, 64>(next, f.A + z * f.sA + (int64_t)kn * n + kn, 0, 0, acc);
+  }
 }
 
 // U[i][j] = X[n-1-i][n-1-j] for i <= j, 0 below the diagonal (OutT = float:
@@ -927,6 +888,17 @@ __global__ void fact_chunk_sub_kernel(const double* P, int64_t sP, int64_t sPc, 
 __global__ void fill_kernel(double* p, int64_t count, double v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   for (; i < count; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
+}
+
+// A first attempt's state: every matrix active at one damp, flags, tickets and step marks clear
+// (one launch where two copies and a fill took 12 us of a small factorization).
+__global__ void fact_init_kernel(int* clear, int64_t count, double* damp, int* active, int batch, double damp0) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) clear[i] = 0;
+  if (i < batch) {
+    damp[i] = damp0;
+    active[i] = 1;
+  }
 }
 
 __global__ void fill_i32_kernel(int* p, int64_t count, int v) {
@@ -1157,17 +1129,22 @@ static const AheadStreams* ahead_streams(hipStream_t st) {
   return &(g_ahead[key] = a);
 }
 
-// One factorization attempt of every active matrix at its damp (w.damp_d),
-// raising w.fail[z] on a bad pivot. Stream-ordered, nothing read back.
+// One factorization attempt of every active matrix at its damp (w.damp_d; first: of every matrix
+// at damp0), raising w.fail[z] on a bad pivot. Stream-ordered, nothing
+// read back.
 template <typename T>
 static int fact_attempt(const T* H, int64_t sH, int n, int batch, const int* order, int64_t sO,
-                        void* U, int u_dtype, int64_t sU, const FactWs& w, hipStream_t st) {
+                        void* U, int u_dtype, int64_t sU, const FactWs& w, bool first, double damp0,
+                        hipStream_t st) {
   const size_t nn = (size_t)n * n;
   const int64_t sA = (int64_t)nn;
   double *A = w.A, *X = w.X, *Tm = w.Tm;
   {
-    const int64_t c = fact_clear_ints(n, batch);
-    fill_i32_kernel<<<(unsigned)((c + 255) / 256), 256, 0, st>>>(w.fail, c, 0);
+    const int64_t c = fact_clear_ints(n, batch);  // at least batch
+    if (first)
+      fact_init_kernel<<<(unsigned)((c + 255) / 256), 256, 0, st>>>(w.fail, c, w.damp_d, w.active, batch, damp0);
+    else
+      fill_i32_kernel<<<(unsigned)((c + 255) / 256), 256, 0, st>>>(w.fail, c, 0);
   }
   // Every entry of X that is read is written first: the diagonal-block kernel stores
   // whole 64 x 64 blocks (zeros above their diagonal), each doubling level stores its
@@ -1179,7 +1156,7 @@ static int fact_attempt(const T* H, int64_t sH, int n, int batch, const int* ord
   if (n > 4096) fill_kernel<<<1024, 256, 0, st>>>(X, (int64_t)nn * batch, 0.0);
   // the order check's marks live in the GEMM scratch Tm, which the split outer updates
   // and the doubling GEMMs later overwrite before reading
-  fact_shift_kernel<T><<<batch, 256, 0, st>>>(H, n, sH, order, sO, w.damp_d, w.diag_tmp, w.shift,
+  fact_shift_kernel<T><<<batch, 1024, 0, st>>>(H, n, sH, order, sO, w.damp_d, w.diag_tmp, w.shift,
                                                 w.active, reinterpret_cast<int*>(Tm),
                                                 (int64_t)(2 * nn), w.fail);
   // rows of H staged per block: as many as fit in 16 KB (at least one), up to 8; rows
@@ -1213,7 +1190,9 @@ static int fact_attempt(const T* H, int64_t sH, int n, int batch, const int* ord
   // 28 matrices of n = 3072 15.4 -> 15.1 ms, n = 2048 5.7 -> 5.6 ms). Beside other size
   // classes' work (compact tiles) a second stream per class only took hardware queues and
   // CUs from a large batch.
-  const AheadStreams* ah = (batch <= 4 || !g_compact_tiles) ? ahead_streams(st) : nullptr;
+  // At n <= 1024 the far updates are shorter than the events that would order them (1024 677 ->
+  // 666 us in place, 1280 863 -> 872).
+  const AheadStreams* ah = (batch <= 4 ? n > 1024 : !g_compact_tiles) ? ahead_streams(st) : nullptr;
   hipStream_t aux = ah ? ah->aux : st;
   bool aux_used = false;
   auto join = [&]() -> int {
@@ -1365,9 +1344,7 @@ static int fact_run(const T* H, int64_t sH, int n, int batch, const int* order, 
                     double* damp_used, char* ws, hipStream_t st, int32_t* flags_out = nullptr) {
   const FactWs w = fact_ws(ws, n, batch);
   if (flags_out) {
-    fill_kernel<<<(batch + 255) / 256, 256, 0, st>>>(w.damp_d, batch, damp0);
-    fill_i32_kernel<<<(batch + 255) / 256, 256, 0, st>>>(w.active, batch, 1);
-    if (int e = fact_attempt<T>(H, sH, n, batch, order, sO, U, u_dtype, sU, w, st)) return e;
+    if (int e = fact_attempt<T>(H, sH, n, batch, order, sO, U, u_dtype, sU, w, true, damp0, st)) return e;
     CP_HIP(hipMemcpyAsync(flags_out, w.fail, batch * sizeof(int), hipMemcpyDeviceToDevice, st));
     return CP_OK;
   }
@@ -1382,13 +1359,15 @@ static int fact_run(const T* H, int64_t sH, int n, int batch, const int* order, 
   for (int attempt = 0; attempt < max_tries; ++attempt) {
     // the previous attempt ended with a stream synchronize, so the pinned
     // buffers are free to rewrite
-    for (int z = 0; z < batch; ++z) {
-      damp_h[z] = damp[z];
-      act_h[z] = act[z];
+    if (attempt) {
+      for (int z = 0; z < batch; ++z) {
+        damp_h[z] = damp[z];
+        act_h[z] = act[z];
+      }
+      CP_HIP(hipMemcpyAsync(w.damp_d, damp_h, batch * sizeof(double), hipMemcpyHostToDevice, st));
+      CP_HIP(hipMemcpyAsync(w.active, act_h, batch * sizeof(int), hipMemcpyHostToDevice, st));
     }
-    CP_HIP(hipMemcpyAsync(w.damp_d, damp_h, batch * sizeof(double), hipMemcpyHostToDevice, st));
-    CP_HIP(hipMemcpyAsync(w.active, act_h, batch * sizeof(int), hipMemcpyHostToDevice, st));
-    if (int e = fact_attempt<T>(H, sH, n, batch, order, sO, U, u_dtype, sU, w, st)) return e;
+    if (int e = fact_attempt<T>(H, sH, n, batch, order, sO, U, u_dtype, sU, w, attempt == 0, damp0, st)) return e;
     CP_HIP(hipMemcpyAsync(fail_h, w.fail, batch * sizeof(int), hipMemcpyDeviceToHost, st));
     CP_HIP(hipStreamSynchronize(st));
     for (int z = 0; z < batch; ++z)

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "kq_blocks.h"
+#include "np_sum.h"
 #include "phase_clock.h"
 
 namespace cp {
@@ -282,63 +283,10 @@ __global__ __launch_bounds__(64 * kSumWaves) void err_colsum_kernel(const ErrDev
   }
 }
 
-// --------------------------------------------------------------- pairwise sum
-// numpy's summation of a contiguous float64 array of n values v(i), n % 8 == 0. It reduces in
-// chunks of 8192 values (its ufunc buffer size), adding the chunk sums left to right onto
-// +0.0. Inside a chunk the sum is pairwise: up to 128 values with eight strided accumulators,
-// ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)); longer runs split at n/2 rounded down to a multiple of
-// 8, the two halves summed recursively. (With n % 8 == 0 every run is a multiple of 8, so no
-// run has a remainder.) One workgroup: the chunk's split tree is laid out as a heap (node i,
-// halves 2i and 2i + 1; m splits into at most m/2 + 8, so 8192 values end at level 7), the
-// leaves summed in parallel by 8 lanes each, and the halves added level by level. One lane
-// walking the tree took 167 us for 29 tensors up to n = 3072; this takes 13.
-constexpr int kNpChunk = 8192, kTreeNodes = 256;
-
-template <class V>
-__device__ double pw_sum_block(const V& v, int64_t n, int2* node, double* val) {
-  double s = 0.0;
-  const int t = (int)threadIdx.x;
-  for (int64_t c0 = 0; c0 < n; c0 += kNpChunk) {
-    __syncthreads();
-    if (t == 0) node[1] = make_int2(0, (int)(n - c0 < kNpChunk ? n - c0 : kNpChunk));
-    for (int first = 1; first < kTreeNodes / 2; first *= 2) {
-      __syncthreads();
-      if (t < first) {
-        const int2 p = node[first + t];
-        const int h = p.y > 128 ? p.y / 2 / 8 * 8 : 0;  // 0: a leaf, or absent (y == 0)
-        node[2 * (first + t)] = make_int2(p.x, h);
-        node[2 * (first + t) + 1] = make_int2(p.x + h, h ? p.y - h : 0);
-      }
-    }
-    __syncthreads();
-    for (int i = 1 + t / 8; i < kTreeNodes; i += 32) {
-      const int2 p = node[i];
-      const bool leaf = p.y > 0 && p.y <= 128;
-      double r = 0.0;
-      if (leaf) {
-        const int64_t o = c0 + p.x + t % 8;
-        r = v(o);
-        for (int k = 8; k < p.y; k += 8) r = r + v(o + k);
-      }
-      r = r + __shfl_xor(r, 1);
-      r = r + __shfl_xor(r, 2);
-      r = r + __shfl_xor(r, 4);
-      if (leaf && t % 8 == 0) val[i] = r;
-    }
-    for (int first = kTreeNodes / 4; first >= 1; first /= 2) {
-      __syncthreads();
-      if (t < first && node[first + t].y > 128) val[first + t] = val[2 * (first + t)] + val[2 * (first + t) + 1];
-    }
-    __syncthreads();
-    s = s + val[1];
-  }
-  return s;
-}
-
+// --------------------------------------------------------------- total
 __global__ __launch_bounds__(256) void err_final_kernel(const ErrDev* __restrict__ tab,
                                                         double* __restrict__ out) {
-  __shared__ int2 node[kTreeNodes];
-  __shared__ double val[kTreeNodes];
+  __shared__ NpSumLds lds;
   const ErrDev& T = tab[blockIdx.x];
   double s;
   const double* ce = T.colerr;
@@ -348,15 +296,15 @@ __global__ __launch_bounds__(256) void err_final_kernel(const ErrDev* __restrict
     const int32_t* perm = T.perm;
     const double* wv = T.wvec;
     const int64_t n = T.n;
-    s = pw_sum_block([=](int64_t i) {
+    s = np_sum_block([=](int64_t i) {
       const int64_t c = perm ? perm[i] : i;
       return ce[i] * wv[c < 0 ? c + n : c];
-    }, T.n, node, val);
+    }, T.n, lds);
   } else if (T.qwp) {
     const float* q = T.qwp;
-    s = pw_sum_block([=](int64_t i) { return ce[i] * (double)q[i]; }, T.n, node, val);
+    s = np_sum_block([=](int64_t i) { return ce[i] * (double)q[i]; }, T.n, lds);
   } else {
-    s = pw_sum_block([=](int64_t i) { return ce[i]; }, T.n, node, val);
+    s = np_sum_block([=](int64_t i) { return ce[i]; }, T.n, lds);
   }
   if (threadIdx.x == 0) out[T.slot] = s;
 }
