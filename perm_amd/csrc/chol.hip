@@ -556,8 +556,10 @@ struct DiagLds {
   double L[NB][NB + 1];
 };
 
+// ready(): called by every thread once it has stored its part of inv(L_kk), before L_kk's.
+template <class Ready>
 __device__ __forceinline__ void diag_block(double* A, int64_t sA, double* X, int64_t sX, int n, int k,
-                                           int* fail, int z, DiagLds& lds) {
+                                           int* fail, int z, DiagLds& lds, const Ready& ready) {
   auto& L = lds.L;
   const int nb = min(NB, n - k);
   double* Ak = A + z * sA + (int64_t)k * n + k;
@@ -723,10 +725,13 @@ __device__ __forceinline__ void diag_block(double* A, int64_t sA, double* X, int
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
     const int r = 4 * m + w;
-    if (r < nb && i < nb) {
-      Xk[(int64_t)r * n + i] = i <= r ? L[i][r + 1] : 0.0;
-      Ak[(int64_t)r * n + i] = i <= r ? L[r][i] : 0.0;
-    }
+    if (r < nb && i < nb) Xk[(int64_t)r * n + i] = i <= r ? L[i][r + 1] : 0.0;
+  }
+  ready();
+#pragma unroll
+  for (int m = 0; m < 16; ++m) {
+    const int r = 4 * m + w;
+    if (r < nb && i < nb) Ak[(int64_t)r * n + i] = i <= r ? L[r][i] : 0.0;
   }
   if (i == 0 && bad) atomicOr(&fail[z], 1);
 }
@@ -737,7 +742,7 @@ __global__ __launch_bounds__(256) void fact_diag_kernel(double* A, int64_t sA, d
   __shared__ DiagLds lds;
   const int z = blockIdx.x;
   if (active && !active[z]) return;
-  diag_block(A, sA, X, sX, n, k, fail, z, lds);
+  diag_block(A, sA, X, sX, n, k, fail, z, lds, [] {});
 }
 
 // ---------------------------------------------------------------- fused chain step
@@ -782,10 +787,12 @@ __global__ __launch_bounds__(256, 2) void fact_step_kernel(FactStep f) {
   const GemmArgs inner{f.A + (int64_t)k * n + f.k0, f.A + (int64_t)k * n + f.k0, f.A + (int64_t)k * n + k,
                        n - k, wk, k - f.k0, n, n, n, -1.0, 1.0, f.sA, f.sA, f.sA, 0, 0, 0, 1, 0};
   if (t == 0) {
-    diag_block(f.A, f.sA, f.X, f.sA, n, k, f.fail, z, lds.d);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(&f.done[z], f.step + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    // the panel items wait for the inverse alone: L_kk is stored after the flag
+    diag_block(f.A, f.sA, f.X, f.sA, n, k, f.fail, z, lds.d, [&] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __syncthreads();
+      if (threadIdx.x == 0) __hip_atomic_store(&f.done[z], f.step + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    });
     return;
   }
   if (k > f.k0) {
