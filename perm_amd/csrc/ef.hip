@@ -9,8 +9,8 @@
 //   LT     [n][nrow] u8   stored codes (q - lo) per visited column
 //   dlT/mlT [n/sub][nrow] f32  committed grid step / offset per storage sub-block
 //
-// Sweep (exact mode): one wavefront owns a stripe of 32 rows and walks the
-// visiting order in 64-column blocks. Left-looking: before a block is swept,
+// Sweep (exact mode): one wavefront (several in calls of fewer rows) owns a stripe
+// of 32, 16 or 4 rows and walks the visiting order in 64-column blocks. Left-looking: before a block is swept,
 // each of its elements receives the updates of all earlier columns,
 //     t -= e_jj * U[jj][k]   (float32 multiply, then subtract, jj ascending),
 // which is exactly the order in which ef.py:213 applies them, so the sweep is
