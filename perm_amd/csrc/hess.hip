@@ -398,7 +398,9 @@ __global__ __launch_bounds__(256) void hess_tri_reduce_kernel(const HessJobs job
 // one 64 x 64 tile of the lower triangle over all rows: its eight waves take a row range each,
 // stage their rows through LDS of their own (no barrier; rows of 192 bytes keep the
 // transposed reads conflict-free), and their sums are added in wave order in LDS. Bound by the
-// latency of a wave's stages: [2048, 1024] 31.2 -> 15.5 us a call, host work included.
+// launch and the panels' way from L2 through LDS (512 KB a workgroup at [2048, 1024]), not by
+// load latency (four stages in flight instead of two: 15.2 -> 16.0): [2048, 1024] 31.2 -> 15.5 us
+// a call, host work included.
 constexpr int SW = 8;                    // waves
 constexpr int SROW = 64 * 2 + 64;        // bytes per padded panel row
 constexpr int SPANEL = KS * SROW;        // 6 KB
