@@ -29,6 +29,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int HT = 128;  // f32 kernel: H tile edge
 constexpr int KT = 32;   // f32 kernel: rows of X per step
+constexpr int kFlush = 8;  // f32 and few-rows kernels: stages summed in one chain, 256 rows
 
 // Row of the 32x32 MFMA result held by register v of lane l (column = l % 32).
 __device__ __forceinline__ int mfma32_row(int v, int l) { return 8 * (v >> 2) + 4 * (l >> 5) + (v & 3); }
@@ -405,6 +406,7 @@ constexpr int SW = 8;                    // waves
 constexpr int SROW = 64 * 2 + 64;        // bytes per padded panel row
 constexpr int SPANEL = KS * SROW;        // 6 KB
 constexpr int SPITCH = 64 + 1;           // floats per row of a wave's sums
+static_assert(kFlush % 2 == 0, "the loop takes two stages at a time");
 
 __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJobs jobs, int64_t N, int d) {
   union Lds {
@@ -424,13 +426,16 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
   const int64_t stages_all = (N + KS - 1) / KS, per = (stages_all + SW - 1) / SW;
   const int64_t r0 = min(N, wv * per * KS), r1 = min(N, (wv + 1) * per * KS);
   const int ns = (int)((r1 - r0 + KS - 1) / KS);
-  f32x16 acc[2][2];
+  // sums of kFlush stages, and their running total: one chain over all N / 8 rows is further from
+  // the float64 sums than the 256 x 256 tiles' shorter splits ([12288, 1024] of unit normals
+  // 1.22e-7 against 9.6e-8, 5.9e-8 with the totals; 51.3 us either way)
+  f32x16 acc[2][2], tot[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[x][y][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) acc[x][y][v] = tot[x][y][v] = 0.0f;
   if (ns > 0) {
     const uint32_t rowb = 2u * (uint32_t)d;
     const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(X + r0 * d), 0, (int)((r1 - r0) * rowb), 0x00020000);
@@ -492,6 +497,15 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
     for (int s = 0; s < ns; s += 2) {
       stage(s, g0);
       if (s + 1 < ns) stage(s + 1, g1);
+      if (s % kFlush == kFlush - 2 || s + 2 >= ns) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            tot[x][y] += acc[x][y];
+            acc[x][y] = 0.0f;
+          }
+      }
     }
   }
   __syncthreads();  // every wave is done with its staging area
@@ -500,7 +514,7 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
 #pragma unroll
     for (int y = 0; y < 2; ++y)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) lds.sum[wv][32 * x + mfma32_row(v, l)][32 * y + (l & 31)] = acc[x][y][v];
+      for (int v = 0; v < 16; ++v) lds.sum[wv][32 * x + mfma32_row(v, l)][32 * y + (l & 31)] = tot[x][y][v];
   __syncthreads();
   // entry (r, c) of the tile: H plus the waves' sums in order, at (i, j) and, as H leaves
   // symmetric, at (j, i); a diagonal tile's entries above the diagonal are its mirror's
@@ -543,7 +557,6 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
 // part: split s of tile k goes to slot (s, k) for hess_f32_reduce_kernel. part == nullptr
 // (one split): the workgroup adds its tile into H, above the diagonal transposed.
 constexpr int FCH = KT * HT / 256;  // floats per thread, panel and stage
-constexpr int kFlush = 8;           // stages summed in one chain: 256 rows
 
 __global__ __launch_bounds__(256, 2) void hess_f32_kernel(const float* __restrict__ X, int64_t N, int d,
                                                           int ntiles, int splits, int64_t rows_per_split,

@@ -35,7 +35,8 @@ def test_few_rows_bf16(hs, N, d, jobs):
     """bf16 batches of few rows at the edges of the 64-column tiles, the 32-row stages and the
     eight waves' row ranges (some without rows), on both sides of the rule that picks the
     kernel: H's lower triangle plus the products, mirrored, whatever its upper triangle held.
-    2^-20 as for float32: chains of at most 1536 rows, then eight sums."""
+    2^-20 as for float32: chains of at most 256 rows and of their sums, then eight waves' sums
+    (at most 512 rows and 25 splits on the other side of the rule)."""
     print(f"few rows N={N} d={d} jobs={jobs}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(N * 1000 + d)
     Xs = [torch.randn((N, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(jobs)]
@@ -47,6 +48,24 @@ def test_few_rows_bf16(hs, N, d, jobs):
         want = (H0 + torch.tril(H0, -1).T).double() + X.double().T @ X.double()
         assert torch.equal(H, H.T)
         assert float(torch.linalg.norm(H.double() - want) / torch.linalg.norm(want)) < 2.0 ** -20
+
+
+@pytest.mark.parametrize("N,d,jobs", [(8192, 1024, 1), (6144, 512, 2), (16384, 128, 1), (2049, 64, 1)])
+def test_few_rows_bf16_sums_short_chains(hs, N, d, jobs):
+    """The few-rows kernel sums a wave's rows in chains of 256. Row 0 gives every entry 2^28
+    (spacing 32), the others 1 each: 16 of them, an MFMA's, are half a spacing, so a chain that
+    holds 2^28 loses what it adds, at most its own 256 rows, and each later addition (a chain's
+    sum onto the wave's, eight waves' sums) at most half a spacing. One chain over a wave's
+    N / 8 rows would lose nearly all of them."""
+    print(f"short chains N={N} d={d} jobs={jobs}", flush=True)
+    X = torch.ones((N, d), device="cuda")
+    X[0] = 2.0 ** 14
+    Hs = hs.xtx_accumulate_many([X.to(torch.bfloat16) for _ in range(jobs)],
+                                [torch.zeros((d, d), device="cuda") for _ in range(jobs)])
+    chains = -(-N // 8 // 256)
+    for H in Hs:
+        lost = float((H.double() - (2.0 ** 28 + N - 1)).abs().max())
+        assert lost <= 256 + 16 * (chains + 8), lost
 
 
 @pytest.mark.parametrize("N,d", [(1, 1), (31, 63), (128, 129), (129, 127), (257, 130), (4097, 65),
