@@ -775,14 +775,31 @@ static int f32_splits(int64_t N, int64_t d, int64_t* rows_per_split) {
 
 constexpr size_t kTileBytes = (size_t)BT * BT * sizeof(float);
 
-// The few-rows kernel for launches whose 64 x 64 tiles run in one round (one workgroup per CU)
-// and whose activations are small. Measured against the 256 x 256 tiles, us: [2048, 1024] 15.5 /
-// 31.2, [8192, 1024] 36 / 49, [12288, 1024] 51 / 55, [16384, 1024] 65 / 61, [32768, 384] 97 / 110,
-// [65536, 512] 209 / 123, [100, 1384] 13 / 60, [8192, 1384] 49 / 48; past one round: 4 x
-// [2048, 1024] 43 / 37, [2048, 3072] 76 / 52.
+// Whether a launch of cn jobs takes the few-rows kernel: its 64 x 64 tiles run in one round (one
+// workgroup per CU) and its predicted time is below the row splits'. In microseconds past the
+// launches: a workgroup walks all N rows at 2.4 per 1024, more as tiles share the L2s (several
+// jobs share no rows and wear on them sooner than one), and 0.7 more per unit where X is past one
+// XCD's 4 MB L2 and its rows end inside a 128-byte line (a panel's 128-byte rows then take two;
+// up to 128 columns the other panel of the workgroup uses the rest). The splits take their rounds
+// of stages, their partial tiles' way through memory, and in the reduction a chain of one load
+// per split for each 16 columns of a thread's 64. On 650 shapes (d = 8-1408, 64-131072 rows,
+// 1-200 jobs) the line picks no kernel more than 2 % slower than the other; few-rows / splits, us:
+// [2048, 1024] 17 / 31, [12288, 1024] 51 / 54, [16384, 1024] 66 / 61, [14000, 896] 52 / 58,
+// [14000, 880] 70 / 58, [49152, 256] 138 / 218, [131072, 64] 332 / 314, [65536, 8] 160 / 71,
+// 4 x [8192, 512] 47 / 51, 6 x 64 / 48, 5 x [49152, 256] 145 / 95, 64 x [32768, 64] 122 / 165.
 static bool few_rows(int cn, int64_t N, int64_t d) {
-  const int64_t t64 = (d + 63) / 64;
-  return t64 * (t64 + 1) / 2 * cn <= 256 && N * d <= (int64_t)3 << 22;
+  const int64_t t64 = (d + 63) / 64, tiles = t64 * (t64 + 1) / 2 * cn;
+  if (tiles > 256 || N * d > (int64_t)1 << 29) return false;  // also: buffer offsets below 2^31
+  const int64_t T = (d + BT - 1) / BT, units = T * (T + 1) / 2 * cn;
+  int64_t rps = 0;
+  const int s = pick_splits((int)units, N, d, &rps);
+  const double load = cn == 1 ? (double)tiles / 600.0 : (double)(tiles * tiles) / (200.0 * 200.0);
+  const bool torn = d > 128 && d % 64 && 2 * N * d * cn > (4 << 20);
+  const double few = 0.0024 * (double)N * (1.0 + load + (torn ? 0.7 : 0.0));
+  const double stages = (double)((units * s + 255) / 256) * ((double)(rps / KS) + 6.0);
+  const int64_t chains = (d + 15) / 16 < 4 ? (d + 15) / 16 : 4;
+  const double sums = s > 1 ? (double)s * (0.26 * (double)chains + 0.02 * (double)units) : 0.0;
+  return few <= 1.0 + 0.5 * stages + sums;
 }
 
 // Workspace of one bf16 launch of cn jobs (0 when it runs as one split).

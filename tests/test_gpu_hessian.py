@@ -30,7 +30,9 @@ def test_xtx_matches_closed_form(hs, dtype, N, d):
 
 @pytest.mark.parametrize("N,d,jobs", [(1, 8, 1), (31, 64, 2), (33, 72, 3), (255, 136, 1), (257, 200, 1),
                                       (2049, 1400, 1), (12288, 1024, 1), (12289, 1024, 1),
-                                      (300, 1024, 2)])
+                                      (300, 1024, 2), (4096, 512, 6), (8192, 512, 6),
+                                      (32768, 64, 3), (196608, 64, 1), (49152, 256, 1),
+                                      (49152, 256, 5), (8192, 16, 1), (65536, 8, 1)])
 def test_few_rows_bf16(hs, N, d, jobs):
     """bf16 batches of few rows at the edges of the 64-column tiles, the 32-row stages and the
     eight waves' row ranges (some without rows), on both sides of the rule that picks the
