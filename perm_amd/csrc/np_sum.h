@@ -7,9 +7,10 @@
 //
 // The chunk's split tree is laid out as a heap (node i, halves 2i and 2i + 1; a run of m
 // values splits into at most m/2 + 8, so 8192 end by level 7), its leaves are summed in
-// parallel by 8 lanes each, and the halves added level by level. Walked by one lane, the tree
-// is a chain of dependent loads (objective totals of 29 tensors up to n = 3072: 167 us, 13
-// here; the damping shift of one n = 1024 / 2000 matrix: 19 / 40 us, 8 / 13 here).
+// parallel by 8 lanes each, and the halves added level by level, over as many levels as the
+// chunk can reach (all seven for 32 values: 4.3 us, 2.0 so). Walked by one lane, the tree is a
+// chain of dependent loads (objective totals of 29 tensors up to n = 3072: 167 us, 13 here; the
+// damping shift of one n = 1024 / 2000 matrix: 19 / 40 us, 8 / 13 here).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -31,9 +32,12 @@ __device__ double np_sum_block(const V& v, int64_t n, NpSumLds& lds) {
   double s = 0.0;
   const int t = (int)threadIdx.x, groups = (int)blockDim.x / 8;
   for (int64_t c0 = 0; c0 < n; c0 += kNpChunk) {
+    const int count = (int)(n - c0 < kNpChunk ? n - c0 : kNpChunk);
+    int last = 1;  // first node of the last level
+    for (int m = count; m > 128; m = m / 2 + 8) last *= 2;
     __syncthreads();
-    if (t == 0) node[1] = make_int2(0, (int)(n - c0 < kNpChunk ? n - c0 : kNpChunk));
-    for (int first = 1; first < kTreeNodes / 2; first *= 2) {
+    if (t == 0) node[1] = make_int2(0, count);
+    for (int first = 1; first < last; first *= 2) {
       __syncthreads();
       if (t < first) {
         const int2 p = node[first + t];
@@ -43,8 +47,9 @@ __device__ double np_sum_block(const V& v, int64_t n, NpSumLds& lds) {
       }
     }
     __syncthreads();
-    for (int i = 1 + t / 8; i < kTreeNodes + 1; i += groups) {  // the same trips for every lane of a wave
-      const int2 p = i < kTreeNodes ? node[i] : make_int2(0, 0);
+    for (int i0 = 0; i0 < 2 * last; i0 += groups) {  // the same trips for every lane of a wave
+      const int i = i0 + t / 8;
+      const int2 p = i > 0 && i < 2 * last ? node[i] : make_int2(0, 0);
       const bool leaf = p.y > 0 && p.y <= 128;
       const int whole = p.y / 8 * 8;
       double r = 0.0;
@@ -61,7 +66,7 @@ __device__ double np_sum_block(const V& v, int64_t n, NpSumLds& lds) {
         val[i] = r;
       }
     }
-    for (int first = kTreeNodes / 4; first >= 1; first /= 2) {
+    for (int first = last / 2; first >= 1; first /= 2) {
       __syncthreads();
       if (t < first && node[first + t].y > 128) val[first + t] = val[2 * (first + t)] + val[2 * (first + t) + 1];
     }

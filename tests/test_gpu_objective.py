@@ -70,6 +70,22 @@ def test_tensor_err_at_tile_edges(ob, tt, nrow, n):
     assert many == [Po.tensor_err(other, "Q6_K", None), want]
 
 
+@pytest.mark.parametrize("n", [32, 96, 128, 160, 256, 288, 512, 544, 1024, 1056, 2080])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_tensor_err_narrow_and_ragged_widths(ob, n, dtype):
+    """Widths whose gather puts several rows into a workgroup pass (up to 512 columns, some
+    with threads left over) and one, 33 rows over two 32-row tiles; totals whose tree ends at
+    each of its first levels, n = 128 m being the largest of a level."""
+    _say(f"narrow {dtype} [33, {n}]")
+    x = heavy_tailed(33, n, seed=n)
+    x = x.astype(np.float16) if dtype == "f16" else x
+    rng = np.random.default_rng(n)
+    wvec, perm = 10.0 ** rng.uniform(-3, 5, n), rng.permutation(n)
+    for rows in (None, 31):
+        want = Po.tensor_err(x, "Q8_0", None, perm=perm, wvec=wvec, rows_sample=rows)
+        assert ob.tensor_err(x, "Q8_0", None, perm=perm, wvec=wvec, rows_sample=rows) == want
+
+
 def _one_tree(v):
     """Pairwise sum of v as one tree (numpy's order only up to 8192 values)."""
     n = len(v)
