@@ -57,13 +57,14 @@ struct ErrDev {
 // consecutive columns' indices in registers over the tile's rows, so an entry costs its
 // gathered load and a quarter of a 16-byte store. (One thread per four entries of a
 // (largest tensor, tensors) grid, reading and checking its indices for every row, took
-// 238 us for 29 tensors of 1 M - 16.8 M entries; this takes 138, 3.5 TB/s of f16 in and f32 out.) Negative indices count from
-// the end, as numpy's do; indices still out of range read element 0 and flag the tensor, whose
-// result becomes NaN.
+// 238 us for 29 tensors of 1 M - 16.8 M entries; this takes 138, 3.5 TB/s of f16 in and f32
+// out.) Negative indices count from the end, as numpy's do; indices still out of range read
+// element 0 and flag the tensor, whose result becomes NaN.
 constexpr int kGatherRows = 32, kGatherCols = 1024;
 
+// Rows i0, i0 + step, ... below i1, columns j .. j + 3.
 template <bool F16>
-__device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int j) {
+__device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int step, int j) {
   const int n = T.n;
   const GU16 x16 = (GU16)T.x;
   const GF32 x32 = (GF32)T.x;
@@ -91,19 +92,19 @@ __device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int
   float4* out = reinterpret_cast<float4*>(T.xs + j);
   constexpr int U = 8;  // rows in flight
   int i = i0;
-  for (; i + U <= i1; i += U) {
+  for (; i1 - i > (U - 1) * step; i += U * step) {
     float v[U][4];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t o = row_of(i + u);
+      const int64_t o = row_of(i + u * step);
 #pragma unroll
       for (int q = 0; q < 4; ++q) v[u][q] = F16 ? half_value(x16[o + c[q]]) : x32[o + c[q]];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      out[(int64_t)(i + u) * (n / 4)] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
+      out[(int64_t)(i + u * step) * (n / 4)] = make_float4(v[u][0], v[u][1], v[u][2], v[u][3]);
   }
-  for (; i < i1; ++i) {
+  for (; i < i1; i += step) {
     const int64_t o = row_of(i);
     float v[4];
 #pragma unroll
@@ -136,14 +137,17 @@ __global__ __launch_bounds__(256) void err_gather_kernel(const ErrDev* __restric
     }
   }
   const int ct = (n + kGatherCols - 1) / kGatherCols, rt = blk / ct;
-  const int j = (blk - rt * ct) * kGatherCols + 4 * (int)threadIdx.x;
-  if (j >= n) return;  // n % 32 == 0: the four columns exist together
+  // up to 512 columns leave half the threads or more over: they take rows of their own (32
+  // columns walked by 8 of 256 threads, [64, 32]: 6.4 us; 3.1 so)
+  const int w = n / 4 < 256 ? n / 4 : 256, step = 256 / w, r = (int)threadIdx.x / w;
+  const int j = (blk - rt * ct) * kGatherCols + 4 * ((int)threadIdx.x - r * w);
+  if (r >= step || j >= n) return;  // n % 32 == 0: the four columns exist together
   const int64_t i0 = (int64_t)rt * kGatherRows;
   const int i1 = (int)(T.R - i0 < kGatherRows ? T.R : i0 + kGatherRows);
   if (T.x_f16)
-    gather_tile<true>(T, (int)i0, i1, j);
+    gather_tile<true>(T, (int)i0 + r, i1, step, j);
   else
-    gather_tile<false>(T, (int)i0, i1, j);
+    gather_tile<false>(T, (int)i0 + r, i1, step, j);
 }
 
 // Workgroups of one tensor's gather.
