@@ -712,18 +712,20 @@ __global__ __launch_bounds__(64, 2) void ef_sweep_rows_kernel(const SweepTask* _
   }
 }
 
-// Wait (bounded) until *done > c, the count of the stripe's blocks complete so far, and
-// return that count. The producing wave releases the count at workgroup scope after
-// its error stores, so the acquire here orders this wave's later reads of those errors.
-// The bound is ``limit`` sleeps of s_sleep 8 (about 512 clocks each): the default
+// Wait (bounded) until *done > c, the count of the stripe's blocks (quarter blocks in the quad
+// sweep) complete so far, and return that count. The producing wave releases the count at
+// workgroup scope after its error stores, so the acquire here orders this wave's later reads of
+// those errors. The bound is ``limit`` times 512 clocks, in sleeps of SLEEP x 64: the default
 // 2^16 is about 14 ms at 2.4 GHz, far above any wait the schedule makes (one block's
 // sweep). Past it the wave sets bit 0 of the call's status word (read by the host,
 // which then rejects the call's bytes) and goes on with one more block rather than
 // spin for ever, so every wave still ends.
-__device__ __forceinline__ int wait_blocks(int* done, int c, int limit, int* status, int lane) {
+template <int SLEEP>
+__device__ __forceinline__ int wait_count(int* done, int c, int limit, int* status, int lane) {
+  static_assert(8 % SLEEP == 0, "whole sleeps per 512 clocks");
   int v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-  for (int spins = 0; v <= c && spins < limit; ++spins) {
-    __builtin_amdgcn_s_sleep(8);
+  for (int64_t spins = 0; v <= c && spins < (int64_t)limit * (8 / SLEEP); ++spins) {
+    __builtin_amdgcn_s_sleep(SLEEP);
     v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   v = __builtin_amdgcn_readfirstlane(v);
@@ -768,7 +770,7 @@ __global__ __launch_bounds__(64 * W, 2) void ef_sweep_pipe_kernel(const SweepTas
     const int i1 = b * 64;
     StripeVec<RS> t = stage_block<RS>(tk, i1, rr, l, s);
     for (int c = 0; c < b;) {
-      const int avail = min(wait_blocks(&done, c, wait_limit, status, l), b);
+      const int avail = min(wait_count<8>(&done, c, wait_limit, status, l), b);
       cross_range<RS>(tk, i1, rr, l, t, c * 64, avail * 64);
       c = avail;
     }
@@ -906,22 +908,6 @@ __device__ __forceinline__ void quad_quarter(const SweepTask& tk, int i1, int l,
   }
 }
 
-// Wait (bounded, as wait_blocks, in sleeps of about 64 clocks) until more than c quarter
-// blocks are complete; returns their count.
-__device__ __forceinline__ int wait_quarters(int* done, int c, int limit, int* status, int lane) {
-  int v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-  for (int64_t spins = 0; v <= c && spins < 4 * (int64_t)limit; ++spins) {
-    __builtin_amdgcn_s_sleep(1);
-    v = __hip_atomic_load(done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  v = __builtin_amdgcn_readfirstlane(v);
-  if (v <= c) {
-    if (lane == 0) __hip_atomic_fetch_or(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return c + 1;
-  }
-  return v;
-}
-
 // Wave w of a stripe owns blocks w, w + W, ...; every element receives its updates one at a
 // time in ascending column order, and blocks complete in order, as in ef_sweep_pipe_kernel.
 template <int NMAX>
@@ -1009,7 +995,7 @@ __global__ __launch_bounds__(64 * kQuadWaves, 2) void ef_sweep_quad_kernel(
       load(2 * q0, u[0]);
       for (int q = q0; q < q1; ++q) {
         load(2 * q + 1, u[1]);
-        if (avail <= q) avail = wait_quarters(&s.done, q, wait_limit, status, l);
+        if (avail <= q) avail = wait_count<1>(&s.done, q, wait_limit, status, l);
         apply(2 * q, u[0]);
         load(q + 1 < q1 ? 2 * q + 2 : 2 * q + 1, u[0]);  // past the end: valid rows, never used
         apply(2 * q + 1, u[1]);
