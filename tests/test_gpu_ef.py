@@ -377,9 +377,45 @@ def test_quad_stripes_bit_exact(ef, waves, monkeypatch):
         bad = np.nonzero((raw.cpu().numpy() != want_raw).any(1))[0]
         assert bad.size == 0, f"{tt}: rows {bad} differ"
         assert np.array_equal(rec.cpu().numpy(), want_rec, equal_nan=True)  # 1e6 overflows fp16
-        rs, wv = (ctypes.c_int * 1)(), (ctypes.c_int * 1)()
-        _lib.load().cp_ef_last_sweep(ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(wv, ctypes.c_void_p))
-        assert rs[0] == 4
+        assert _last_sweep() == (_lib.CP_EF_EXACT, 4, min(int(waves), W.shape[1] // 64))
+
+
+def _last_sweep():
+    """(mode, rows per stripe, waves per stripe) of the calling thread's last sweep launch."""
+    rs, wv = (ctypes.c_int * 1)(), (ctypes.c_int * 1)()
+    mode = _lib.load().cp_ef_last_sweep(ctypes.cast(rs, ctypes.c_void_p), ctypes.cast(wv, ctypes.c_void_p))
+    return mode, rs[0], wv[0]
+
+
+@pytest.mark.parametrize("tt", TYPES)
+@pytest.mark.parametrize("waves", ["1", "8"])
+def test_quad_stripes_non_finite_rows(ef, tt, waves, monkeypatch):
+    """Infinities and NaN, in the weights (in the first column visited, in the middle of a
+    block's later quarters, in the last block) and, from there, in the propagated errors, and a
+    non-finite U: the four-row stripes give the 16-row kernel's bytes and reconstructions, rows
+    beside them in a stripe included."""
+    n = 1024
+    (W, _, qw, H, order, U), = _oracle_items([(22, n, tt, 81)])
+    for row, place, v in ((0, 0, np.inf), (1, 40, np.nan), (2, 300, -np.inf), (5, 991, np.nan),
+                          (6, 1023, np.inf), (9, 512, np.inf), (9, 555, -np.inf)):
+        W[row, order[place]] = v
+    U_bad = U.copy()
+    U_bad[200, 700], U_bad[64, 65] = np.inf, np.nan
+    for what, Um in (("weights", U), ("U", U_bad)):
+        _say(f"quad non-finite {what}: {tt}, waves {waves}")
+        item = {"ttype": tt, "x": torch.from_numpy(W).cuda(), "qw": torch.from_numpy(qw).cuda(),
+                "U": torch.from_numpy(Um).cuda(),
+                "order": torch.from_numpy(order.astype(np.int32)).cuda()}
+        got = {}
+        for rows in ("4", "16"):
+            monkeypatch.setenv("CP_EF_SWEEP_ROWS", rows)
+            monkeypatch.setenv("CP_EF_SWEEP_WAVES", waves)
+            (raw, rec), = ef.ef_encode_dev([item], 2)
+            assert _last_sweep() == (_lib.CP_EF_EXACT, int(rows), int(waves))
+            got[rows] = raw.cpu().numpy(), rec.cpu().numpy()
+        bad = np.nonzero((got["4"][0] != got["16"][0]).any(1))[0]
+        assert bad.size == 0, f"{what}: rows {bad} differ"
+        assert np.array_equal(got["4"][1], got["16"][1], equal_nan=True)
 
 
 def _codes(tt, raw, nrow, n):
@@ -548,9 +584,11 @@ def test_factor_async_equals_blocking(ef):
 
 @pytest.mark.parametrize("n,batch", [(3072, 4), (1000, 3)])
 def test_factor_compact_tiles_give_the_same_factor(ef, n, batch):
-    """cp_chol_compact_tiles(1) (every fp64 GEMM on 64 x 64 tiles, as the concurrent
-    size-class driver queues them) gives bit-identical U: each output element sums its K
-    range in the same order whatever the tile."""
+    """cp_chol_compact_tiles(1) (separate launches instead of the fused steps, no look-ahead
+    stream for batches of more than four, no 128 x 128 GEMM tiles; as the concurrent size-class
+    driver queues wide or large classes) gives bit-identical U. At these sizes no product takes
+    a 128 x 128 tile: the 32 x 32 and 64 x 64 tiles are compared by the batch of five against
+    one of test_fused_steps_give_the_separate_launches_factor at n = 3072."""
     lib = _lib.load()
     _say(f"compact tiles n={n} batch={batch}")
     Hb = torch.from_numpy(np.stack([correlated_hessian(n, 2 * n, seed=40 + s)

@@ -71,12 +71,13 @@ def test_few_rows_bf16_sums_short_chains(hs, N, d, jobs):
 
 
 @pytest.mark.parametrize("N,d", [(1, 1), (31, 63), (128, 129), (129, 127), (257, 130), (4097, 65),
-                                 (1000, 387)])
+                                 (1000, 387), (1000, 2900)])
 def test_float32_tiles_add_to_any_h(hs, N, d):
     """float32 X at the edges of the 128-column tiles, the 32-row stages and the row splits (one
-    split and several), on an H that is not symmetric: both triangles keep their own values
-    under the sum. 2^-20 bounds it: sums of at most 4097 products in chains of at most 128
-    rows' MFMA steps and 33 splits stay well below 1e-6 of their norm."""
+    split and several; 2900 columns are 276 tiles, so one split of 32 stages and four chains),
+    on an H that is not symmetric: both triangles keep their own values under the sum. 2^-20
+    bounds it: sums of at most 4097 products in chains of at most 256 rows' MFMA steps and 33
+    splits stay well below 1e-6 of their norm."""
     print(f"float32 tiles N={N} d={d}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(N * 1000 + d)
     X = torch.randn((N, d), generator=g, device="cuda")
