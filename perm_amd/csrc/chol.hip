@@ -318,10 +318,11 @@ static bool pairs_aligned(const double* p, int ld, int64_t s1, int64_t s2) {
   return aligned(p, 16) && !(ld & 1) && !(s1 & 1) && !(s2 & 1);
 }
 
-// The calling thread's GEMM tile policy (cp_chol_compact_tiles): 0 picks the fastest tile
-// for a GPU the factorization has to itself; 1 keeps every GEMM at 64 x 64, whose blocks
-// (112 VGPRs, 36 KB of LDS) fit on a CU beside two EF sweep waves per SIMD, where the
-// 128 x 128 tile (234-256 VGPRs, 69-72 KB) waits for whole CUs to drain.
+// The calling thread's launch policy (cp_chol_compact_tiles): 0 picks the fastest tiles and
+// launches for a GPU the factorization has to itself; 1 takes no GEMM tile above 64 x 64, whose
+// blocks (112 VGPRs, 36 KB of LDS; the 32 x 32 ones less) fit on a CU beside two EF sweep waves
+// per SIMD, where the 128 x 128 tile (234-256 VGPRs, 69-72 KB) waits for whole CUs to drain, no
+// fused chain steps, and a look-ahead stream only for at most kFusedBatch matrices.
 static thread_local int g_compact_tiles = 0;
 
 // Fused chain steps for calls of at most this many matrices, and the bounded wait of a

@@ -16,10 +16,10 @@
 #include <hip/hip_runtime.h>
 
 #include "cp_host.h"
+#include "np_sum.h"
 
 namespace cp {
 
-constexpr int kNpChunk = 8192;  // elements per inner-loop call of numpy's reduction
 constexpr int kLeaf = 128;
 
 struct SqErrTerms {
