@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
     for (int s = 0; s < ns; s += 2) {
       stage(s, g0);
       if (s + 1 < ns) stage(s + 1, g1);
-      if (s % kFlush == kFlush - 2 || s + 2 >= ns) {
+      if (s % kFlush == kFlush - 2 && s + 2 < ns) {
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
@@ -514,7 +514,7 @@ __global__ __launch_bounds__(64 * SW, 2) void hess_bf16_small_kernel(const HessJ
 #pragma unroll
     for (int y = 0; y < 2; ++y)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) lds.sum[wv][32 * x + mfma32_row(v, l)][32 * y + (l & 31)] = tot[x][y][v];
+      for (int v = 0; v < 16; ++v) lds.sum[wv][32 * x + mfma32_row(v, l)][32 * y + (l & 31)] = tot[x][y][v] + acc[x][y][v];
   __syncthreads();
   // entry (r, c) of the tile: H plus the waves' sums in order, at (i, j) and, as H leaves
   // symmetric, at (j, i); a diagonal tile's entries above the diagonal are its mirror's
