@@ -7,8 +7,8 @@
 // split a workgroup adds its finished tile into H itself (one writer per
 // element); with several, each split stores its tile into a workspace slot of
 // its own and one reduction pass adds the splits' tiles to H in split order
-// (H + ((p0 + p1) + p2 ...)). The same X therefore gives the same H bit for
-// bit, run after run.
+// (H + ((p0 + p1) + p2 ...), the f32 path in groups of 16 splits). The same X
+// therefore gives the same H bit for bit, run after run.
 //
 //  bf16: lower-triangle 256 x 256 tiles on v_mfma_f32_32x32x16_bf16, operands
 //        read transposed from LDS (hess_bf16_tri_kernel), then a pass that
@@ -681,10 +681,12 @@ __global__ __launch_bounds__(256, 2) void hess_f32_kernel(const float* __restric
   if (!diag) add(j0, i0, [&](int r) { return tl[c * (HT + 4) + r]; });
 }
 
-// The row splits' tiles summed in split order, p_0 + p_1 + ..., and added to H at (i, j) and
-// (j, i), over 32 x 32 blocks of the lower triangle (blockIdx.x, row order; small blocks, so a
-// narrow H with many splits still fills the chip); the mirror goes through LDS so both sides
-// are coalesced.
+// The row splits' tiles summed in split order, by groups (p_0 + ... + p_15) + (p_16 + ...) + ...,
+// and added to H at (i, j) and (j, i), over 32 x 32 blocks of the lower triangle (blockIdx.x, row
+// order; small blocks, so a narrow H with many splits still fills the chip); the mirror goes
+// through LDS so both sides are coalesced.
+constexpr int kSplitGroup = 16;
+
 __global__ __launch_bounds__(256) void hess_f32_reduce_kernel(float* __restrict__ H, int d, int ntiles,
                                                               int splits, const float* __restrict__ part) {
   __shared__ float tl[32][33];
@@ -696,13 +698,36 @@ __global__ __launch_bounds__(256) void hess_f32_reduce_kernel(float* __restrict_
   const int ti = bi / 4, tj = bj / 4;
   const int64_t slot = (int64_t)ntiles * (HT * HT);  // floats between one split's tiles
   const float* p = part + (int64_t)(ti * (ti + 1) / 2 + tj) * (HT * HT) + ((bi % 4) * 32 + rt) * HT + (bj % 4) * 32 + c;
+  // groups of kSplitGroup splits, and their running total: one chain over a narrow H's splits (up
+  // to 512) is further from the float64 sums than fewer, longer splits ([16384, 200] of values
+  // about 1: 9.4e-8 in 32 splits, 1.5e-7 in a chain of 128, 5.2e-8 so; [65536, 64] 1.5e-7, 3.0e-7,
+  // 7.8e-8, and 85 -> 54 us a call with a group's loads in flight)
   float s[4];
+  int k0 = 0;
+  for (; k0 + kSplitGroup <= splits; k0 += kSplitGroup) {
+    float v[kSplitGroup][4];  // a group's loads all in flight
 #pragma unroll
-  for (int q = 0; q < 4; ++q) s[q] = p[8 * q * HT];
+    for (int k = 0; k < kSplitGroup; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[k][q] = p[(k0 + k) * slot + 8 * q * HT];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int k = 1; k < kSplitGroup; ++k) v[0][q] += v[k][q];
+      s[q] = k0 ? s[q] + v[0][q] : v[0][q];
+    }
+  }
+  if (k0 < splits) {
+    float g[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) g[q] = p[k0 * slot + 8 * q * HT];
 #pragma unroll 4
-  for (int k = 1; k < splits; ++k)
+    for (int k = k0 + 1; k < splits; ++k)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s[q] += p[k * slot + 8 * q * HT];
+      for (int q = 0; q < 4; ++q) g[q] += p[k * slot + 8 * q * HT];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) s[q] = k0 ? s[q] + g[q] : g[q];
+  }
   const int j = bj * 32 + c;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {

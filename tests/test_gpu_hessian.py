@@ -89,6 +89,20 @@ def test_float32_tiles_add_to_any_h(hs, N, d):
     assert torch.equal(hs.xtx_accumulate(X), hs.xtx_accumulate(X).T)
 
 
+@pytest.mark.parametrize("N,d", [(65536, 64), (16384, 200), (8192, 129)])
+def test_float32_splits_are_summed_in_groups(hs, N, d):
+    """Narrow float32 X is split every 128 rows, and the splits' tiles are added in groups of
+    16. Split 0 gives every entry 2^28 (spacing 32), each other split 4: what is added to the
+    2^28 one split at a time is lost, 4 for each of the first group's 15, while a later group's
+    64 is a whole number of spacings. One chain over all splits would lose all of them."""
+    print(f"float32 split groups N={N} d={d}", flush=True)
+    X = torch.zeros((N, d), device="cuda")
+    X[::128] = 2.0
+    X[0] = 2.0 ** 14
+    lost = (hs.xtx_accumulate(X).double() - (2.0 ** 28 + 4 * (N // 128 - 1))).abs()
+    assert float(lost.max()) <= 4 * 15
+
+
 def test_accumulates_in_place(hs):
     g = torch.Generator(device="cuda").manual_seed(0)
     X1 = torch.randn((3000, 512), generator=g, device="cuda").to(torch.bfloat16)
