@@ -9,8 +9,8 @@
 // values splits into at most m/2 + 8, so 8192 end by level 7), its leaves are summed in
 // parallel by 8 lanes each, and the halves added level by level, over as many levels as the
 // chunk can reach (all seven for 32 values: 4.3 us, 2.0 so). Walked by one lane, the tree is a
-// chain of dependent loads (objective totals of 29 tensors up to n = 3072: 167 us, 13 here; the
-// damping shift of one n = 1024 / 2000 matrix: 19 / 40 us, 8 / 13 here).
+// chain of dependent loads (objective totals of 29 tensors up to n = 3072: 167 us, 10 here; the
+// damping shift of one n = 1024 matrix: 19 us, 7 here).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
