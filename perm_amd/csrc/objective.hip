@@ -10,13 +10,14 @@
 //            order of numpy's d2.sum(0) over a C-contiguous array, so the result is
 //            bit-identical
 //   final    +0.0 plus numpy's pairwise sum of colerr * w (the order of a
-//            contiguous float64 .sum()), one lane per tensor
+//            contiguous float64 .sum()), one workgroup per tensor
 // col_log_rms(x, row_step) is the per-column float64 sum of squares in row chunks
 // (a sequential chain per chunk, the chunk sums added in order), then
 // log(sqrt(acc / nrow) + 1e-12).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "kq_blocks.h"
@@ -62,10 +63,11 @@ struct ErrDev {
 // element 0 and flag the tensor, whose result becomes NaN.
 constexpr int kGatherRows = 32, kGatherCols = 1024;
 
-// Rows i0, i0 + step, ... below i1, columns j .. j + 3.
-template <bool F16>
-__device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int step, int j) {
-  const int n = T.n;
+// Rows i0, i0 + steps, ... below i1, columns j .. j + 3. NARROW false: steps is 1 (its own code:
+// a step in a register took the 1024-wide tiles 137 -> 142 us).
+template <bool F16, bool NARROW>
+__device__ __forceinline__ void gather_tile(const ErrDev& T, int i0, int i1, int steps, int j) {
+  const int n = T.n, step = NARROW ? steps : 1;
   const GU16 x16 = (GU16)T.x;
   const GF32 x32 = (GF32)T.x;
   const GI32 perm = (GI32)T.perm, rows = (GI32)T.rows;
@@ -144,10 +146,17 @@ __global__ __launch_bounds__(256) void err_gather_kernel(const ErrDev* __restric
   if (r >= step || j >= n) return;  // n % 32 == 0: the four columns exist together
   const int64_t i0 = (int64_t)rt * kGatherRows;
   const int i1 = (int)(T.R - i0 < kGatherRows ? T.R : i0 + kGatherRows);
+  const auto tile = [&](auto f16) {
+    constexpr bool F16 = decltype(f16)::value;
+    if (step > 1)
+      gather_tile<F16, true>(T, (int)i0 + r, i1, step, j);
+    else
+      gather_tile<F16, false>(T, (int)i0, i1, 1, j);
+  };
   if (T.x_f16)
-    gather_tile<true>(T, (int)i0 + r, i1, step, j);
+    tile(std::true_type());
   else
-    gather_tile<false>(T, (int)i0 + r, i1, step, j);
+    tile(std::false_type());
 }
 
 // Workgroups of one tensor's gather.
